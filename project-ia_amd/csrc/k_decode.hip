@@ -416,30 +416,28 @@ __device__ __forceinline__ uint32_t host_word(const uint32_t* p) {
 // x = embd[token] (reference model.c:1027-1068); out-of-range tokens are
 // clamped (the host validates the tokens it submits; a device-fed token is an
 // argmax result, always < vocab).  The token comes from device memory, or,
-// with host (pinned memory: token, position, -, whether they hold) and its
-// last word set, from there, and is then stored to tok and pos for the
-// kernels behind: once per workgroup, as each read crosses the link.  With
-// two 4-byte copies ahead of the step and one behind it for the logits, one
-// layer of Llama-3-8B at position 2047 with an 8192-token vocabulary took
-// 158 us from call to return; with these reads and k_to_host 144 (150 with
-// the words read by every thread).
+// with host (pinned memory: token, position), from there, and is then stored
+// to tok and pos for the kernels behind: once per workgroup, as each read
+// crosses the link.  With two 4-byte copies ahead of the step and one behind
+// it for the logits, one layer of Llama-3-8B at position 2047 with an
+// 8192-token vocabulary took 158 us from call to return; with these reads and
+// k_to_host 144 (150 with the words read by every thread).
 __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, uint32_t* tok, uint32_t* pos,
                                                const uint32_t* host, uint32_t vocab, uint32_t dim4,
                                                float4* __restrict__ x) {
     __shared__ uint32_t t_s;
     if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        bool fed = false;
+        uint32_t t;
         if (host) {
             t = host_word(host);
             const uint32_t hp = host_word(host + 1);
-            fed = host_word(host + 3) != 0;
-            if (fed && blockIdx.x == 0) {  // (no workgroup reads them here)
+            if (blockIdx.x == 0) {  // (no workgroup reads them here)
                 *tok = t;
                 *pos = hp;
             }
+        } else {
+            t = *tok;
         }
-        if (!fed) t = *tok;
         t_s = t < vocab ? t : vocab - 1;
     }
     __syncthreads();

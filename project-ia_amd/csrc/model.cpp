@@ -65,10 +65,11 @@ struct ModelPlan {
     float* kv = nullptr;
     size_t kv_layer_floats = 0;
     hipStream_t stream = nullptr;
-    hipGraphExec_t step_graph = nullptr;     // decode step, host-fed token/pos
-    hipGraphExec_t gen_graph = nullptr;      // decode step + greedy feedback + pos advance
+    hipGraphExec_t step_graph = nullptr;     // decode step, token/pos from the pinned words
+    hipGraphExec_t loop_graph = nullptr;     // decode step, token/pos in device memory (sampled generation)
+    hipGraphExec_t gen_graph = nullptr;      // the same + greedy feedback + pos advance
     void* sample_ws = nullptr;               // device workspace of sampled generation
-    uint32_t* pinned = nullptr;              // host staging: token, pos, 0, whether the step graph takes them
+    uint32_t* pinned = nullptr;              // host staging: token, pos, 0
     float* pinned_logits = nullptr;          // host staging for the logits llama_forward returns
     // Batched prefill (llama_forward with seq_len > 1), allocated at its
     // first use: row buffers for pf_rows tokens and the GEMM workspace.
@@ -90,6 +91,7 @@ void plan_destroy(CtxState* st) {
     if (!p) return;
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     if (p->step_graph) (void)hipGraphExecDestroy(p->step_graph);
+    if (p->loop_graph) (void)hipGraphExecDestroy(p->loop_graph);
     if (p->gen_graph) (void)hipGraphExecDestroy(p->gen_graph);
     if (p->arena) (void)hipFree(p->arena);
     if (p->sample_ws) (void)hipFree(p->sample_ws);
@@ -153,13 +155,19 @@ static q_tensor* make_view(q_context* ctx, size_t offset, uint32_t n0, uint32_t 
 // ---------------------------------------------------------------------------
 // Decode step enqueue (all kernels on p->stream)
 // ---------------------------------------------------------------------------
+// Where a step's token and position come from: the pinned words (host), or
+// device memory, where the step itself (greedy) or a kernel behind it (loop)
+// leaves the next ones.
+enum class Feed { host, loop, greedy };
+
 // One decode step in 7 kernels per layer: Q|K|V from fp32 x (RMSNorm and
 // digits in the prologue, RoPE and KV-cache stores in the epilogue),
 // attention (3 kernels: the reference's clamped polynomial exp needs the
 // global max before any exponential; the combine emits o's digits), Wo +
 // residual, W_gate|W_up from fp32 x1 (FFN RMSNorm in the prologue, SwiGLU
 // in the epilogue, fp32 h out), W_down from fp32 h + residual.
-static hipError_t enqueue_step_fused(ModelPlan* p, bool feedback) {
+static hipError_t enqueue_step_fused(ModelPlan* p, Feed feed) {
+    const bool feedback = feed == Feed::greedy;
     const q_llama_config& c = p->cfg;
     hipStream_t s = p->stream;
     hipError_t e;
@@ -169,7 +177,8 @@ static hipError_t enqueue_step_fused(ModelPlan* p, bool feedback) {
         if (e != hipSuccess) return e;   \
     } while (0)
     const uint32_t nblk_d = c.dim / 32;
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, c.vocab_size, c.dim, p->x, s));
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size, c.dim,
+                      p->x, s));
     for (uint32_t l = 0; l < c.n_layers; ++l) {
         const LayerDev& L = p->layers[l];
         float* kvl = p->kv + (size_t)l * p->kv_layer_floats;
@@ -248,8 +257,9 @@ static hipError_t enqueue_step_fused(ModelPlan* p, bool feedback) {
     return hipSuccess;
 }
 
-static hipError_t enqueue_step(ModelPlan* p, bool feedback) {
-    if (p->fused) return enqueue_step_fused(p, feedback);
+static hipError_t enqueue_step(ModelPlan* p, Feed feed) {
+    if (p->fused) return enqueue_step_fused(p, feed);
+    const bool feedback = feed == Feed::greedy;
     const q_llama_config& c = p->cfg;
     hipStream_t s = p->stream;
     hipError_t e;
@@ -258,7 +268,8 @@ static hipError_t enqueue_step(ModelPlan* p, bool feedback) {
         e = (x);                         \
         if (e != hipSuccess) return e;   \
     } while (0)
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, c.vocab_size, c.dim, p->x, s));
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size, c.dim,
+                      p->x, s));
     GemvDecode dec;
     dec.pos = p->pos;
     dec.cos_tab = p->cos_tab;
@@ -319,9 +330,9 @@ static hipError_t enqueue_step(ModelPlan* p, bool feedback) {
     return hipSuccess;
 }
 
-static q_error_code capture(ModelPlan* p, bool feedback, hipGraphExec_t* out) {
+static q_error_code capture(ModelPlan* p, Feed feed, hipGraphExec_t* out) {
     QH_TRY(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
-    const hipError_t e = enqueue_step(p, feedback);
+    const hipError_t e = enqueue_step(p, feed);
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(p->stream, &g);
     if (e != hipSuccess) {
@@ -526,8 +537,9 @@ static q_error_code bind_kv(ModelPlan* p, const q_context* ctx) {
     if (p->kv != kv) {
         QH_TRY(hipStreamSynchronize(p->stream));
         if (p->step_graph) QH_TRY(hipGraphExecDestroy(p->step_graph));
+        if (p->loop_graph) QH_TRY(hipGraphExecDestroy(p->loop_graph));
         if (p->gen_graph) QH_TRY(hipGraphExecDestroy(p->gen_graph));
-        p->step_graph = p->gen_graph = nullptr;
+        p->step_graph = p->loop_graph = p->gen_graph = nullptr;
         p->kv = kv;
     }
     return Q_OK;
@@ -808,11 +820,11 @@ q_error_code llama_forward(q_llama_model* __restrict__ model, q_context* __restr
     QH_TRY_CODE(check_kv(p, ctx));
     QH_TRY_CODE(bind_kv(p, ctx));
     if (seq_len == 1) {
-        if (!p->step_graph) QH_TRY_CODE(capture(p, false, &p->step_graph));
+        if (!p->step_graph) QH_TRY_CODE(capture(p, Feed::host, &p->step_graph));
         QH_TRY(hipStreamSynchronize(p->stream));  // pinned staging is reused each step
         p->pinned[0] = tokens[0];
         p->pinned[1] = pos;
-        p->pinned[3] = 1;  // the step's embedding launch reads them from here
+        // (the step's embedding launch reads them from there)
         QH_TRY(hipGraphLaunch(p->step_graph, p->stream));
     } else {
         QH_TRY_CODE(prefill_alloc(p));
@@ -893,7 +905,7 @@ q_error_code qh_llama_generate(q_llama_model* model, q_context* ctx, uint32_t to
     if (!p) return Q_ERR_INVALID_ARG;
     QH_TRY_CODE(check_kv(p, ctx));
     QH_TRY_CODE(bind_kv(p, ctx));
-    if (!p->gen_graph) QH_TRY_CODE(capture(p, true, &p->gen_graph));
+    if (!p->gen_graph) QH_TRY_CODE(capture(p, Feed::greedy, &p->gen_graph));
     QH_TRY(hipStreamSynchronize(p->stream));
     p->pinned[0] = token;
     p->pinned[1] = pos;
@@ -940,7 +952,7 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     if (!p) return Q_ERR_INVALID_ARG;
     QH_TRY_CODE(check_kv(p, ctx));
     QH_TRY_CODE(bind_kv(p, ctx));
-    if (!p->step_graph) QH_TRY_CODE(capture(p, false, &p->step_graph));
+    if (!p->loop_graph) QH_TRY_CODE(capture(p, Feed::loop, &p->loop_graph));
     const uint32_t V = p->cfg.vocab_size;
     if (!p->sample_ws) {
         const size_t wb = sample_workspace_bytes(V);
@@ -958,7 +970,6 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     p->pinned[0] = token;
     p->pinned[1] = pos;
     p->pinned[2] = 0;
-    p->pinned[3] = 0;  // the step graph takes token and position from the device
     QH_TRY(hipMemcpyAsync(p->tok, &p->pinned[0], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->pos, &p->pinned[1], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->hist_n, &p->pinned[2], 4, hipMemcpyHostToDevice, p->stream));
@@ -967,7 +978,7 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     QH_TRY(hipEventCreate(&e1));
     QH_TRY(hipEventRecord(e0, p->stream));
     for (uint32_t i = 0; i < n_steps; ++i) {
-        QH_TRY(hipGraphLaunch(p->step_graph, p->stream));
+        QH_TRY(hipGraphLaunch(p->loop_graph, p->stream));
         sp.r = sample_draw();
         QH_TRY(launch_sample(p->logits, sp, p->sample_ws, p->tok, p->stream));
         QH_TRY(launch_token_feedback(p->tok, p->pos, p->hist, p->hist_n, p->hist_cap, p->stream));

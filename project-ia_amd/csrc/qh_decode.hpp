@@ -30,8 +30,8 @@ size_t attention_scratch_floats(uint32_t n_heads, uint32_t max_seq);
 size_t attention_n_chunks(uint32_t max_seq);
 
 hipError_t launch_swiglu_prep(const float* g, const float* u, uint32_t N, float* m_out, uint4* xd, hipStream_t s);
-// host: null, or 4 words of pinned memory (token, position, -, fed): when fed
-// is set the launch takes token and position from there and stores them.
+// host: null (token and position are in device memory), or two words of pinned
+// memory (token, position) that the launch reads and stores to tok and pos.
 hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host, uint32_t vocab,
                         uint32_t dim, float* x, hipStream_t s);
 // n device floats to pinned host memory.
