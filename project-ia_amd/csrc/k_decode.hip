@@ -413,9 +413,16 @@ __device__ __forceinline__ uint32_t host_word(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// x = embd[token] (reference model.c:1027-1068); out-of-range tokens are
-// clamped (the host validates the tokens it submits; a device-fed token is an
-// argmax result, always < vocab).  The token comes from device memory, or,
+// The nearest index below n.
+__host__ __device__ constexpr uint32_t bounded(uint32_t i, uint32_t n) { return i < n ? i : n - 1u; }
+static_assert(bounded(0u, 1u) == 0u && bounded(2055u, 2056u) == 2055u && bounded(2056u, 2056u) == 2055u &&
+                  bounded(0xFFFFFFFFu, 2056u) == 2055u,
+              "a stray token or position must stay inside its table");
+
+// x = embd[token] (reference model.c:1027-1068).  Token and position are
+// bounded here, ahead of every kernel that addresses by them (the position
+// steers the KV-cache stores): the host validates what it submits and the
+// device loops stay in range, so the bound only acts on a stray word.  The token comes from device memory, or,
 // with host (pinned memory: token, position), from there, and is then stored
 // to tok and pos for the kernels behind: once per workgroup, as each read
 // crosses the link.  With two 4-byte copies ahead of the step and one behind
@@ -423,22 +430,17 @@ __device__ __forceinline__ uint32_t host_word(const uint32_t* p) {
 // 8192-token vocabulary took 158 us from call to return; with these reads and
 // k_to_host 144 (150 with the words read by every thread).
 __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, uint32_t* tok, uint32_t* pos,
-                                               const uint32_t* host, uint32_t vocab, uint32_t dim4,
-                                               float4* __restrict__ x) {
+                                               const uint32_t* host, uint32_t vocab, uint32_t max_seq,
+                                               uint32_t dim4, float4* __restrict__ x) {
     __shared__ uint32_t t_s;
     if (threadIdx.x == 0) {
-        uint32_t t;
-        if (host) {
-            t = host_word(host);
-            const uint32_t hp = host_word(host + 1);
-            if (blockIdx.x == 0) {  // (no workgroup reads them here)
-                *tok = t;
-                *pos = hp;
-            }
-        } else {
-            t = *tok;
+        const uint32_t t = host ? host_word(host) : *tok;
+        if (blockIdx.x == 0) {  // (no other workgroup reads pos, nor tok with host)
+            const uint32_t p = host ? host_word(host + 1) : *pos;
+            if (host) *tok = t;
+            if (host || p >= max_seq) *pos = bounded(p, max_seq);
         }
-        t_s = t < vocab ? t : vocab - 1;
+        t_s = bounded(t, vocab);
     }
     __syncthreads();
     const uint32_t t = t_s;
@@ -447,10 +449,10 @@ __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, 
 }
 
 hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host, uint32_t vocab,
-                        uint32_t dim, float* x, hipStream_t s) {
-    if (dim % 4 != 0) return hipErrorInvalidValue;
+                        uint32_t max_seq, uint32_t dim, float* x, hipStream_t s) {
+    if (dim % 4 != 0 || vocab == 0 || max_seq == 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_embed, dim3((dim / 4 + 255) / 256), dim3(256), 0, s, reinterpret_cast<const float4*>(embd), tok,
-                       pos, host, vocab, dim / 4, reinterpret_cast<float4*>(x));
+                       pos, host, vocab, max_seq, dim / 4, reinterpret_cast<float4*>(x));
     return hipGetLastError();
 }
 

@@ -177,8 +177,8 @@ static hipError_t enqueue_step_fused(ModelPlan* p, Feed feed) {
         if (e != hipSuccess) return e;   \
     } while (0)
     const uint32_t nblk_d = c.dim / 32;
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size, c.dim,
-                      p->x, s));
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size,
+                      c.max_seq_len, c.dim, p->x, s));
     for (uint32_t l = 0; l < c.n_layers; ++l) {
         const LayerDev& L = p->layers[l];
         float* kvl = p->kv + (size_t)l * p->kv_layer_floats;
@@ -268,8 +268,8 @@ static hipError_t enqueue_step(ModelPlan* p, Feed feed) {
         e = (x);                         \
         if (e != hipSuccess) return e;   \
     } while (0)
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size, c.dim,
-                      p->x, s));
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size,
+                      c.max_seq_len, c.dim, p->x, s));
     GemvDecode dec;
     dec.pos = p->pos;
     dec.cos_tab = p->cos_tab;
