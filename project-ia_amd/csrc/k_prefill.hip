@@ -137,21 +137,23 @@ hipError_t launch_rope_kv_rows(float* Q, const float* K, const float* V, const f
 //    all-zero or non-finite row), and split as hi = rn(k'), lo = rn(k' - hi)
 //    (the subtraction is exact in fp32): 22 significant bits of every
 //    element within 2^17 of the row maximum, steps of 2^-24 (of k') below
-//    that.  With each row goes a flag: the key's V row holds a NaN or an
-//    infinity (its P.V terms must then be formed even where e_j = 0, as
-//    0 * v_j is NaN).
+//    that.
 //  * Values: one exponent per KV head, from the largest finite |v| over its
 //    keys (so that max|v'| lies in [2^14, 2^15)), the same hi/lo split, and
 //    stored transposed per 64-key stage, [dim][64 keys], the keys of each
 //    32-key half in the order the P.V fragments read them (positions
-//    8g + 4s + r hold key 16s + 4g + r).
+//    8g + 4s + r hold key 16s + 4g + r).  A NaN or an infinity is stored as 0
+//    and noted: per dimension, the first key that holds one.  A query that
+//    attends that key gets NaN there, whatever its e_j (0 * v_j is NaN); one
+//    that ends before it never meets it, though its tile's stages hold the
+//    key's row.
 // Layout (256-byte aligned pieces): K halfs [n_kv][max_seq][hi 128 | lo
-// 128]; int32 2e + flag [n_kv][max_seq]; float partial max|v| [n_kv]
-// [max_seq / 8]; int32 V exponent [n_kv]; V halfs [n_kv][stages][hi | lo]
-// [128][64].
+// 128]; int32 e [n_kv][max_seq]; float partial max|v| [n_kv][max_seq / 8];
+// int32 V exponent [n_kv]; int32 first non-finite key [n_kv][128]; V halfs
+// [n_kv][stages][hi | lo][128][64].
 // ---------------------------------------------------------------------------
 struct KhlLayout {
-    size_t meta, vmax, vexp, vt, bytes;
+    size_t kexp, vmax, vexp, vbad, vt, bytes;
     uint32_t n_wa, n_st;  // partials per head (8 keys each), 64-key stages per head
 };
 
@@ -161,10 +163,11 @@ __host__ __device__ inline KhlLayout khl_layout(uint32_t n_kv, uint32_t max_seq)
     const size_t rows = (size_t)n_kv * max_seq;
     L.n_wa = (max_seq + 7) / 8;
     L.n_st = (max_seq + 63) / 64;
-    L.meta = al(rows * 2 * kPHd * 2);
-    L.vmax = L.meta + al(rows * 4);
+    L.kexp = al(rows * 2 * kPHd * 2);
+    L.vmax = L.kexp + al(rows * 4);
     L.vexp = L.vmax + al((size_t)n_kv * L.n_wa * 4);
-    L.vt = L.vexp + al((size_t)n_kv * 4);
+    L.vbad = L.vexp + al((size_t)n_kv * 4);
+    L.vt = L.vbad + al((size_t)n_kv * kPHd * 4);
     L.bytes = L.vt + (size_t)n_kv * L.n_st * 64 * 2 * kPHd * 2;
     return L;
 }
@@ -182,8 +185,11 @@ __device__ __forceinline__ int split_exp(float m) {
     return (m > 0.0f && m <= FLT_MAX) ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
 }
 
-// Key rows, their flags, and each 8-row group's largest finite |v|: one
-// 32-lane half of a wave per row, one float4 of K and of V per lane.
+constexpr int kNoKey = 0x7FFFFFFF;
+
+// Key rows, and each 8-row group's largest finite |v|: one 32-lane half of a
+// wave per row, one float4 of K and of V per lane.  The first workgroup of a
+// head clears its notes of non-finite keys.
 __global__ __launch_bounds__(256) void k_prefill_khl(const float* __restrict__ kv, uint32_t n_keys, uint32_t max_seq,
                                                      void* __restrict__ khl, KhlLayout L) {
     __shared__ float red[4];
@@ -197,16 +203,10 @@ __global__ __launch_bounds__(256) void k_prefill_khl(const float* __restrict__ k
         vx = *reinterpret_cast<const float4*>(kv + row * (2 * kPHd) + kPHd + 4 * c);
     }
     const float va[4] = {fabsf(vx.x), fabsf(vx.y), fabsf(vx.z), fabsf(vx.w)};
-    bool vbad = false;
     float mv = 0.0f;  // largest finite |v|
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const bool fin = va[i] <= FLT_MAX;
-        vbad |= !fin;
-        mv = fin ? fmaxf(mv, va[i]) : mv;
-    }
-    const uint64_t vb = __ballot(vbad);
-    const bool row_vbad = ((threadIdx.x & 32) ? (uint32_t)(vb >> 32) : (uint32_t)vb) != 0u;
+    for (int i = 0; i < 4; ++i) mv = va[i] <= FLT_MAX ? fmaxf(mv, va[i]) : mv;
+    if (blockIdx.x == 0 && threadIdx.x < kPHd) khl_at<int>(khl, L.vbad)[kvh * kPHd + threadIdx.x] = kNoKey;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) mv = fmaxf(mv, __shfl_xor(mv, off));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mv;
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void k_prefill_khl(const float* __restrict__ k
         _Float16* dst = khl_at<_Float16>(khl, 0) + row * (2 * kPHd) + 4 * c;
         *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(hi);
         *reinterpret_cast<uint2*>(dst + kPHd) = *reinterpret_cast<const uint2*>(lo);
-        if (c == 0) khl_at<int>(khl, L.meta)[row] = 2 * e + (row_vbad ? 1 : 0);
+        if (c == 0) khl_at<int>(khl, L.kexp)[row] = e;
     }
     __syncthreads();
     if (threadIdx.x == 0)
@@ -241,7 +241,8 @@ __device__ __forceinline__ uint32_t vt_pos(uint32_t r) {
 }
 
 // V of one 64-key stage of one KV head, scaled by the head's exponent,
-// split into hi/lo and transposed (through LDS); keys past n_keys are 0.
+// split into hi/lo and transposed (through LDS); keys past n_keys are 0, and
+// so are non-finite elements, whose keys are noted.
 __global__ __launch_bounds__(256) void k_prefill_vt(const float* __restrict__ kv, uint32_t n_keys, uint32_t max_seq,
                                                     void* __restrict__ khl, KhlLayout L) {
     __shared__ float red[4];
@@ -270,7 +271,11 @@ __global__ __launch_bounds__(256) void k_prefill_vt(const float* __restrict__ kv
         const uint32_t pos = vt_pos(r);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float v = ldexpf(xs[e], ev);
+            float v = ldexpf(xs[e], ev);
+            if (!(fabsf(xs[e]) <= FLT_MAX)) {
+                v = 0.0f;
+                atomicMin(khl_at<int>(khl, L.vbad) + kvh * kPHd + 4 * c + e, (int)j);
+            }
             const _Float16 hv = (_Float16)v;
             lt[0][4 * c + e][pos] = hv;
             lt[1][4 * c + e][pos] = (_Float16)(v - (float)hv);
@@ -356,7 +361,7 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
     // 128 bytes per dimension d, chunk c in place c ^ (d / 2 % 8): the 16 lanes
     // that read one chunk of 16 rows cover 64 banks either way.
     __shared__ __attribute__((aligned(1024))) uint8_t lds[2][kAttnStage];
-    __shared__ __attribute__((aligned(256))) int lmeta[2][kAttnKS];  // 2e + V flag of the staged keys
+    __shared__ __attribute__((aligned(256))) int lke[2][kAttnKS];  // the staged keys' exponents
     __shared__ float xmax[2][HG][16], xsum[HG][16];
 
     const uint32_t n_qt = (a.T + 15) / 16;
@@ -377,10 +382,10 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
     const uint32_t n_stages = (n_keys + kAttnKS - 1) / kAttnKS;
     const size_t q_ld = (size_t)a.n_heads * kPHd;
     const KhlLayout L = khl_layout(a.n_kv, a.max_seq);
-    // key rows (hi|lo halfs, 128 floats' worth each), 2e + V flag, the
+    // key rows (hi|lo halfs, 128 floats' worth each), their exponents, the
     // transposed V stages and the head's V exponent
     const float* khbase = khl_at<const float>(a.khl, 0) + (size_t)kvh * a.max_seq * kPHd;
-    const int* kmbase = khl_at<const int>(a.khl, L.meta) + (size_t)kvh * a.max_seq;
+    const int* kebase = khl_at<const int>(a.khl, L.kexp) + (size_t)kvh * a.max_seq;
     const float* vtbase = khl_at<const float>(a.khl, L.vt) + (size_t)kvh * L.n_st * (kPHd * 64);
     const int ev = khl_at<const int>(a.khl, L.vexp)[kvh];
 
@@ -433,14 +438,15 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
             }
     }
 
-    // Stage st of K or V into LDS buffer b, of the keys' 2e + V flags into
-    // lmeta[m].  The K and flag resources end at the tile's last key: rows
-    // past it (zeros, or the rows behind them in the same workspace, whether
-    // or not the range check counts the scalar offset) only meet scores masked
-    // by j <= P below and the zero V parts k_prefill_vt writes past the keys.
-    const rsrc_v rk = make_rsrc(khbase, n_keys * kPHd * 4u), rm = make_rsrc(kmbase, n_keys * 4u);
+    // Stage st of K or V into LDS buffer b, of the keys' exponents into lke[m].
+    // The K and exponent resources end at the tile's last key: rows past it
+    // (zeros, or the rows behind them in the same workspace, whether or not the
+    // range check counts the scalar offset) only meet scores masked by j <= P
+    // below, whose e_j = 0 then meet finite V parts (of later tokens, or zeros
+    // past the prompt).
+    const rsrc_v rk = make_rsrc(khbase, n_keys * kPHd * 4u), re = make_rsrc(kebase, n_keys * 4u);
     const rsrc_v rv = make_rsrc(vtbase, n_stages * kAttnStage);
-    const uint32_t lds0 = lds_address(lds) + wave * 1024u, meta0 = lds_address(lmeta);
+    const uint32_t lds0 = lds_address(lds) + wave * 1024u, ke0 = lds_address(lke);
     // Place i = threadIdx.x + u*NT of a stage: of K, key i/32, place i%32; of
     // V, row i/8, place i%8 (NT/8 rows on, the same turn).
     const uint32_t krow = threadIdx.x >> 5;
@@ -456,8 +462,8 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
         for (uint32_t u = 0; u < kLoads; ++u)
             lds_load16(rv, voff_v, st * kAttnStage + u * NT * 16u, lds0 + b * kAttnStage + u * NT * 16u);
     };
-    auto load_meta = [&](uint32_t st, uint32_t m) {
-        if (wave == 0) lds_load4(rm, lane * 4u, st * (kAttnKS * 4u), meta0 + m * (kAttnKS * 4u));
+    auto load_exp = [&](uint32_t st, uint32_t m) {
+        if (wave == 0) lds_load4(re, lane * 4u, st * (kAttnKS * 4u), ke0 + m * (kAttnKS * 4u));
     };
     // This wave's loads have landed and its LDS reads are done, then everyone's.
     auto arrive = [&]() {
@@ -494,16 +500,16 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
         // follow, they read the products a few cycles too early on one path
         // (the compiler does not pad that edge).
         asm volatile("" : "+v"(r0), "+v"(r1));
-        const int4 e0 = *reinterpret_cast<const int4*>(&lmeta[mb][32 * half + 4 * lg]);
-        const int4 e1 = *reinterpret_cast<const int4*>(&lmeta[mb][32 * half + 16 + 4 * lg]);
-        r0[0] = ldexpf(r0[0], -(eq + (e0.x >> 1)));
-        r0[1] = ldexpf(r0[1], -(eq + (e0.y >> 1)));
-        r0[2] = ldexpf(r0[2], -(eq + (e0.z >> 1)));
-        r0[3] = ldexpf(r0[3], -(eq + (e0.w >> 1)));
-        r1[0] = ldexpf(r1[0], -(eq + (e1.x >> 1)));
-        r1[1] = ldexpf(r1[1], -(eq + (e1.y >> 1)));
-        r1[2] = ldexpf(r1[2], -(eq + (e1.z >> 1)));
-        r1[3] = ldexpf(r1[3], -(eq + (e1.w >> 1)));
+        const int4 e0 = *reinterpret_cast<const int4*>(&lke[mb][32 * half + 4 * lg]);
+        const int4 e1 = *reinterpret_cast<const int4*>(&lke[mb][32 * half + 16 + 4 * lg]);
+        r0[0] = ldexpf(r0[0], -(eq + e0.x));
+        r0[1] = ldexpf(r0[1], -(eq + e0.y));
+        r0[2] = ldexpf(r0[2], -(eq + e0.z));
+        r0[3] = ldexpf(r0[3], -(eq + e0.w));
+        r1[0] = ldexpf(r1[0], -(eq + e1.x));
+        r1[1] = ldexpf(r1[1], -(eq + e1.y));
+        r1[2] = ldexpf(r1[2], -(eq + e1.z));
+        r1[3] = ldexpf(r1[3], -(eq + e1.w));
     };
 
     // Row max over the 16 keys of d (scores of keys jb .. jb+15).
@@ -534,7 +540,7 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
     f4v acc[8];
     float sum = 0.0f;
     const uint32_t vat = li * 128u + 16u * ((4u * half + lg) ^ (li >> 1));  // the wave's chunk of dimension li
-    auto pv32 = [&](uint32_t b, uint32_t mb, uint32_t jb, const f4v& d0, const f4v& d1) {
+    auto pv32 = [&](uint32_t b, uint32_t jb, const f4v& d0, const f4v& d1) {
         float e[8];
         if (jb + 32u <= inner) {
             // wave-uniform: every key attended, on the polynomial exp (its
@@ -561,12 +567,10 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
         const float es = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
         sum += es;
         // A 32-key step whose e_j are 0 for every query of the tile adds
-        // exact zeros (0 * v_j for finite v_j): its P.V is skipped.  (The
+        // exact zeros (the V parts are finite): its P.V is skipped.  (The
         // polynomial exp is 0 below about -2.18, so most keys of a peaked
         // score row take no part.)
-        const bool nz = es != 0.0f;
-        if (__ballot(nz || ((lmeta[mb][32 * half + li] | lmeta[mb][32 * half + 16 + li]) & 1) != 0) == 0ull)
-            return;  // wave-uniform
+        if (__ballot(es != 0.0f) == 0ull) return;  // wave-uniform
         h8v ph, pl;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -604,7 +608,7 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
     // Pass 1 alternates the buffers, one barrier a stage; the stage pass 2
     // starts with loads into the next one during the last.
     load_k(0, 0);
-    load_meta(0, 0);
+    load_exp(0, 0);
     if constexpr (kShort) {
         f4v sc[kAttnCacheStages][2];
         // ---- pass 1: scores and row max ----
@@ -614,10 +618,9 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
                 arrive();
                 if (st + 1 < n_stages) {
                     load_k(st + 1, (st + 1) & 1u);
-                    load_meta(st + 1, (st + 1) & 1u);
+                    load_exp(st + 1, (st + 1) & 1u);
                 } else {
                     load_v(0, (st + 1) & 1u);
-                    load_meta(0, (st + 1) & 1u);
                 }
                 // (keys past the tile's last are masked by j <= P)
                 const uint32_t jb = st * kAttnKS + 32 * half;
@@ -634,13 +637,10 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
             if (st < n_stages) {
                 const uint32_t b = (n_stages + st) & 1u;
                 arrive();
-                if (st + 1 < n_stages) {
-                    load_v(st + 1, b ^ 1u);
-                    load_meta(st + 1, b ^ 1u);
-                }
+                if (st + 1 < n_stages) load_v(st + 1, b ^ 1u);
                 const uint32_t jb = st * kAttnKS + 32 * half;
                 if (jb < n_keys)
-                    pv32(b, b, jb, sc[st][0], jb + 16 < n_keys ? sc[st][1] : f4v{0.0f, 0.0f, 0.0f, 0.0f});
+                    pv32(b, jb, sc[st][0], jb + 16 < n_keys ? sc[st][1] : f4v{0.0f, 0.0f, 0.0f, 0.0f});
             }
         }
     } else {
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
             arrive();
             const uint32_t nx = st + 1 < n_stages ? st + 1 : 0u;
             load_k(nx, (st + 1) & 1u);
-            load_meta(nx, (st + 1) & 1u);
+            load_exp(nx, (st + 1) & 1u);
             const uint32_t jb = st * kAttnKS + 32 * half;
             f4v d0, d1;
             scores2(st & 1u, st & 1u, d0, d1);
@@ -673,9 +673,9 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
             arrive();  // V is there; the scores are done with K
             if (st + 1 < n_stages) {
                 load_k(st + 1, bk);
-                load_meta(st + 1, m ^ 1u);
+                load_exp(st + 1, m ^ 1u);
             }
-            if (jb < n_keys) pv32(bk ^ 1u, m, jb, d0, d1);
+            if (jb < n_keys) pv32(bk ^ 1u, jb, d0, d1);
         }
     }
     sum += __shfl_xor(sum, 16);
@@ -697,7 +697,11 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
     sum += xsum[hw][li];
 
     // ---- output: register r of lane l is query 4*(l/16) + r, dimension
-    // 16n + l%16 of tile n; the parts' scales undone exactly first ----
+    // 16n + l%16 of tile n; the parts' scales undone exactly first; NaN where
+    // the query attends a non-finite V ----
+    int bad[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n) bad[n] = khl_at<const int>(a.khl, L.vbad)[kvh * kPHd + 16 * n + li];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const uint32_t i = 4 * lg + (uint32_t)r;
@@ -710,7 +714,7 @@ __global__ __launch_bounds__(128 * HG) __attribute__((amdgpu_waves_per_eu(kShort
 #pragma unroll
             for (int n = 0; n < 8; ++n) {
                 const float v = ldexpf(acc[n][r], -(9 + ev));
-                dst[16 * n] = small ? v / total : v * inv;
+                dst[16 * n] = bad[n] <= (int)(a.pos0 + t) ? __builtin_nanf("") : small ? v / total : v * inv;
             }
         }
     }

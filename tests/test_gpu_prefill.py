@@ -122,6 +122,45 @@ def test_prefill_around_512_keys(qa, tmp_path, n_heads, n_kv, T):
         m.close()
 
 
+# Non-finite token: the last of a tile, inside one (its step straddles other
+# queries' last keys), the first of the next; up to 512 keys and past them.
+@pytest.mark.parametrize("P,T,bad", [(0, 20, 19), (0, 37, 18), (0, 70, 32), (5, 33, 31), (600, 40, 21), (607, 17, 16)])
+@pytest.mark.parametrize("n_heads,n_kv", [(4, 1), (2, 2)])
+def test_prefill_non_finite_token_stays_behind_earlier_queries(qa, tmp_path, n_heads, n_kv, P, T, bad):
+    """A token whose embedding holds an infinity has a non-finite V row.  The
+    tokens before it never attend it: their cache rows are the oracle's, in
+    the layer behind the attention too; the tokens after it attend it, and
+    their rows there are not finite."""
+    h = qa.QorusHeader(vocab=300, dim=128 * n_heads, hidden=512, n_layers=2, n_heads=n_heads, n_kv=n_kv, max_seq=700)
+    path = tmp_path / "nf.qorus"
+    qa.synthetic.write_synthetic_model(path, h, 83)
+    blob = np.fromfile(path, dtype=np.uint8)
+    at = qa.model_layout(h)["token_embd"]
+    blob[at: at + h.vocab * h.dim * 4].view(np.float32).reshape(h.vocab, h.dim)[h.vocab - 1, 3] = np.inf
+    blob.tofile(path)
+    m = qa.Model(path)
+    rng = orc.rng_for(83, n_heads, T)
+    kv = np.zeros((h.n_layers, n_kv, h.max_seq, 2, 128), np.float32)
+    kv[:, :, :P] = rng.standard_normal((h.n_layers, n_kv, P, 2, 128), dtype=np.float32)
+    m.upload_kv(kv)
+    try:
+        toks = [int(t) for t in rng.integers(0, h.vocab - 1, T)]
+        toks[bad] = h.vocab - 1
+        ref = orc.DecodeOracle(blob, kv.copy())
+        for i, t in enumerate(toks[:bad]):
+            ref.fill(t, P + i)
+        m.forward(toks, P)
+        got = m.download_kv().reshape(kv.shape)
+        for l in range(h.n_layers):
+            e = rel_err(got[l, :, P:P + bad], ref.kv[l, :, P:P + bad])
+            assert e <= 1e-4, (l, e)
+        assert not np.isfinite(got[0, :, P + bad, 1]).any()
+        for i in range(bad + 1, T):
+            assert np.isfinite(got[0, :, P + i]).all() and not np.isfinite(got[1, :, P + i, 1]).any(), i
+    finally:
+        m.close()
+
+
 @pytest.mark.parametrize("T", [2, 8, 9, 16, 17])
 def test_prefill_short_prompts(qa, tmp_path, T):
     """Prompts of 2 to 17 tokens at position 0: query rows with fewer than 8
