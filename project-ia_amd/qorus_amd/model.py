@@ -7,7 +7,7 @@ import ctypes as C
 
 import numpy as np
 
-from ._lib import check, lib
+from ._lib import QorusError, check, lib
 from .model_file import QorusHeader
 
 
@@ -45,6 +45,17 @@ class QGenerationState(C.Structure):
                 ("top_p", C.c_float), ("current_pos", C.c_uint32)]
 
 
+class KVView:
+    """The KV cache of a model as a device array [L][n_kv][max_seq][2][head_dim]
+    (float32): torch.as_tensor(view) and other readers of
+    __cuda_array_interface__ keep the view, the view keeps the model, and so
+    the cache outlives every array made from it."""
+
+    def __init__(self, owner, ptr: int, shape):
+        self.owner = owner
+        self.__cuda_array_interface__ = dict(data=(ptr, False), shape=tuple(shape), typestr="<f4", version=2)
+
+
 class Model:
     """A loaded v3 model with an HBM KV cache sized for its max_seq_len."""
 
@@ -76,6 +87,14 @@ class Model:
         out = np.empty(self.n_layers * self.kv_floats_per_layer, dtype=np.float32)
         check(lib().qh_memcpy_dtoh(out.ctypes.data, self.ctx.kv_buffer, out.nbytes), "kv download")
         return out
+
+    def kv_view(self) -> KVView:
+        """The cache for arrays of other libraries.  forward() and the device
+        loops run on a stream of their own: work that fills or reads the cache
+        elsewhere is synchronized by the caller before the next call."""
+        if self._closed:
+            raise QorusError("kv_view: the model is closed")
+        return KVView(self, self.ctx.kv_buffer, (self.n_layers, self.n_kv, self.max_seq, 2, self.head_dim))
 
     def forward(self, tokens, pos: int) -> np.ndarray:
         toks = np.ascontiguousarray(tokens, dtype=np.uint32)

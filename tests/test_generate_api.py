@@ -3,6 +3,7 @@ checked without a GPU: every case fails before the first forward pass."""
 import ctypes as C
 
 import numpy as np
+import pytest
 
 import qorus_amd as qa
 
@@ -56,3 +57,34 @@ def test_q_generate_validation_codes():
     # the order: a zero max_tokens is reported before a bad temperature
     st, keep = state(max_tokens=0, temperature=-1.0)
     assert g(st) == -15
+
+
+def test_kv_view_keeps_the_model_alive():
+    """Arrays made from a model's cache hold its view, and the view the model:
+    the memory is freed only with the last of them."""
+    import gc
+    import weakref
+
+    class Holder(qa.Model):
+        def __init__(self):  # (no model file, no device: the cache's address is a stand-in)
+            self.ctx, self._closed = qa.QContext(), False
+            self.ctx.kv_buffer = 0x1000
+            self.n_layers, self.n_kv, self.max_seq, self.head_dim = 2, 3, 40, 128
+
+        def close(self):
+            self._closed = True
+
+    m = Holder()
+    alive = weakref.ref(m)
+    view = m.kv_view()
+    assert view.__cuda_array_interface__ == dict(data=(0x1000, False), shape=(2, 3, 40, 2, 128), typestr="<f4", version=2)
+    del m
+    gc.collect()
+    assert alive() is not None
+    del view
+    gc.collect()
+    assert alive() is None
+    m = Holder()
+    m.close()
+    with pytest.raises(qa.QorusError):
+        m.kv_view()
