@@ -408,9 +408,11 @@ hipError_t launch_swiglu_prep(const float* g, const float* u, uint32_t N, float*
     return hipGetLastError();
 }
 
-// A word of pinned host memory, read past the caches.
-__device__ __forceinline__ uint32_t host_word(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+// Two words of pinned host memory (8-byte aligned), read past the caches in one
+// crossing of the link.
+__device__ __forceinline__ uint2 host_words(const uint32_t* p) {
+    const uint64_t w = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return make_uint2((uint32_t)w, (uint32_t)(w >> 32));
 }
 
 // The nearest index below n.
@@ -422,23 +424,31 @@ static_assert(bounded(0u, 1u) == 0u && bounded(2055u, 2056u) == 2055u && bounded
 // x = embd[token] (reference model.c:1027-1068).  Token and position are
 // bounded here, ahead of every kernel that addresses by them (the position
 // steers the KV-cache stores): the host validates what it submits and the
-// device loops stay in range, so the bound only acts on a stray word.  The token comes from device memory, or,
-// with host (pinned memory: token, position), from there, and is then stored
-// to tok and pos for the kernels behind: once per workgroup, as each read
-// crosses the link.  With two 4-byte copies ahead of the step and one behind
-// it for the logits, one layer of Llama-3-8B at position 2047 with an
-// 8192-token vocabulary took 158 us from call to return; with these reads and
-// k_to_host 144 (150 with the words read by every thread).
+// device loops stay in range, so the bound only acts on a stray word.  They are
+// in device memory, or, with host and while *looped is 0, in two words of pinned
+// memory, and are then stored for the kernels behind: read once per workgroup,
+// as each read crosses the link.  A device loop over the same graph sets
+// *looped and stays off the link (a graph of its own for it took 2 MB of
+// device memory at the first loop).  With two 4-byte copies ahead of the step
+// and one behind it for the logits, one layer of Llama-3-8B at position 2047
+// with an 8192-token vocabulary took 158 us from call to return; with the
+// reads and k_to_host 144 (150 with the words read by every thread).
 __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, uint32_t* tok, uint32_t* pos,
-                                               const uint32_t* host, uint32_t vocab, uint32_t max_seq,
-                                               uint32_t dim4, float4* __restrict__ x) {
+                                               const uint32_t* host, const uint32_t* looped, uint32_t vocab,
+                                               uint32_t max_seq, uint32_t dim4, float4* __restrict__ x) {
     __shared__ uint32_t t_s;
     if (threadIdx.x == 0) {
-        const uint32_t t = host ? host_word(host) : *tok;
-        if (blockIdx.x == 0) {  // (no other workgroup reads pos, nor tok with host)
-            const uint32_t p = host ? host_word(host + 1) : *pos;
-            if (host) *tok = t;
-            if (host || p >= max_seq) *pos = bounded(p, max_seq);
+        uint32_t t;
+        if (host && *looped == 0) {
+            const uint2 w = host_words(host);
+            t = w.x;
+            if (blockIdx.x == 0) {  // (no workgroup reads them here)
+                *tok = t;
+                *pos = bounded(w.y, max_seq);
+            }
+        } else {
+            t = *tok;
+            if (blockIdx.x == 0 && *pos >= max_seq) *pos = max_seq - 1u;
         }
         t_s = bounded(t, vocab);
     }
@@ -448,11 +458,12 @@ __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, 
         x[i] = embd[(size_t)t * dim4 + i];
 }
 
-hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host, uint32_t vocab,
-                        uint32_t max_seq, uint32_t dim, float* x, hipStream_t s) {
-    if (dim % 4 != 0 || vocab == 0 || max_seq == 0) return hipErrorInvalidValue;
+hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host,
+                        const uint32_t* looped, uint32_t vocab, uint32_t max_seq, uint32_t dim, float* x,
+                        hipStream_t s) {
+    if (dim % 4 != 0 || vocab == 0 || max_seq == 0 || (host && !looped)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_embed, dim3((dim / 4 + 255) / 256), dim3(256), 0, s, reinterpret_cast<const float4*>(embd), tok,
-                       pos, host, vocab, max_seq, dim / 4, reinterpret_cast<float4*>(x));
+                       pos, host, looped, vocab, max_seq, dim / 4, reinterpret_cast<float4*>(x));
     return hipGetLastError();
 }
 

@@ -58,6 +58,7 @@ struct ModelPlan {
     float *scores = nullptr, *part_max = nullptr, *part_sum = nullptr, *o_part = nullptr;
     float *cos_tab = nullptr, *sin_tab = nullptr;
     uint32_t *tok = nullptr, *pos = nullptr, *hist = nullptr, *hist_n = nullptr;
+    uint32_t* looped = nullptr;              // device: 1 while a loop keeps token/pos in device memory
     uint32_t hist_cap = 0;
     float* amax_ws = nullptr;                // multi-workgroup argmax partials
     float* amax_parts = nullptr;             // the LM-head GEMV's argmax partials
@@ -65,11 +66,11 @@ struct ModelPlan {
     float* kv = nullptr;
     size_t kv_layer_floats = 0;
     hipStream_t stream = nullptr;
-    hipGraphExec_t step_graph = nullptr;     // decode step, token/pos from the pinned words
-    hipGraphExec_t loop_graph = nullptr;     // decode step, token/pos in device memory (sampled generation)
-    hipGraphExec_t gen_graph = nullptr;      // the same + greedy feedback + pos advance
+    hipGraphExec_t step_graph = nullptr;     // decode step, token/pos from the pinned words unless *looped
+    hipGraphExec_t gen_graph = nullptr;      // decode step + greedy feedback + pos advance
     void* sample_ws = nullptr;               // device workspace of sampled generation
-    uint32_t* pinned = nullptr;              // host staging: token, pos, 0
+    uint32_t* pinned = nullptr;              // host staging: token, pos, 0, 1
+    bool loop_set = false;                   // *looped is 1 (since the last sampled generation)
     float* pinned_logits = nullptr;          // host staging for the logits llama_forward returns
     // Batched prefill (llama_forward with seq_len > 1), allocated at its
     // first use: row buffers for pf_rows tokens and the GEMM workspace.
@@ -91,7 +92,6 @@ void plan_destroy(CtxState* st) {
     if (!p) return;
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     if (p->step_graph) (void)hipGraphExecDestroy(p->step_graph);
-    if (p->loop_graph) (void)hipGraphExecDestroy(p->loop_graph);
     if (p->gen_graph) (void)hipGraphExecDestroy(p->gen_graph);
     if (p->arena) (void)hipFree(p->arena);
     if (p->sample_ws) (void)hipFree(p->sample_ws);
@@ -155,19 +155,13 @@ static q_tensor* make_view(q_context* ctx, size_t offset, uint32_t n0, uint32_t 
 // ---------------------------------------------------------------------------
 // Decode step enqueue (all kernels on p->stream)
 // ---------------------------------------------------------------------------
-// Where a step's token and position come from: the pinned words (host), or
-// device memory, where the step itself (greedy) or a kernel behind it (loop)
-// leaves the next ones.
-enum class Feed { host, loop, greedy };
-
 // One decode step in 7 kernels per layer: Q|K|V from fp32 x (RMSNorm and
 // digits in the prologue, RoPE and KV-cache stores in the epilogue),
 // attention (3 kernels: the reference's clamped polynomial exp needs the
 // global max before any exponential; the combine emits o's digits), Wo +
 // residual, W_gate|W_up from fp32 x1 (FFN RMSNorm in the prologue, SwiGLU
 // in the epilogue, fp32 h out), W_down from fp32 h + residual.
-static hipError_t enqueue_step_fused(ModelPlan* p, Feed feed) {
-    const bool feedback = feed == Feed::greedy;
+static hipError_t enqueue_step_fused(ModelPlan* p, bool feedback) {
     const q_llama_config& c = p->cfg;
     hipStream_t s = p->stream;
     hipError_t e;
@@ -177,7 +171,7 @@ static hipError_t enqueue_step_fused(ModelPlan* p, Feed feed) {
         if (e != hipSuccess) return e;   \
     } while (0)
     const uint32_t nblk_d = c.dim / 32;
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size,
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, p->looped, c.vocab_size,
                       c.max_seq_len, c.dim, p->x, s));
     for (uint32_t l = 0; l < c.n_layers; ++l) {
         const LayerDev& L = p->layers[l];
@@ -257,9 +251,8 @@ static hipError_t enqueue_step_fused(ModelPlan* p, Feed feed) {
     return hipSuccess;
 }
 
-static hipError_t enqueue_step(ModelPlan* p, Feed feed) {
-    if (p->fused) return enqueue_step_fused(p, feed);
-    const bool feedback = feed == Feed::greedy;
+static hipError_t enqueue_step(ModelPlan* p, bool feedback) {
+    if (p->fused) return enqueue_step_fused(p, feedback);
     const q_llama_config& c = p->cfg;
     hipStream_t s = p->stream;
     hipError_t e;
@@ -268,7 +261,7 @@ static hipError_t enqueue_step(ModelPlan* p, Feed feed) {
         e = (x);                         \
         if (e != hipSuccess) return e;   \
     } while (0)
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feed == Feed::host ? p->pinned : nullptr, c.vocab_size,
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, p->looped, c.vocab_size,
                       c.max_seq_len, c.dim, p->x, s));
     GemvDecode dec;
     dec.pos = p->pos;
@@ -330,9 +323,9 @@ static hipError_t enqueue_step(ModelPlan* p, Feed feed) {
     return hipSuccess;
 }
 
-static q_error_code capture(ModelPlan* p, Feed feed, hipGraphExec_t* out) {
+static q_error_code capture(ModelPlan* p, bool feedback, hipGraphExec_t* out) {
     QH_TRY(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
-    const hipError_t e = enqueue_step(p, feed);
+    const hipError_t e = enqueue_step(p, feedback);
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(p->stream, &g);
     if (e != hipSuccess) {
@@ -537,9 +530,8 @@ static q_error_code bind_kv(ModelPlan* p, const q_context* ctx) {
     if (p->kv != kv) {
         QH_TRY(hipStreamSynchronize(p->stream));
         if (p->step_graph) QH_TRY(hipGraphExecDestroy(p->step_graph));
-        if (p->loop_graph) QH_TRY(hipGraphExecDestroy(p->loop_graph));
         if (p->gen_graph) QH_TRY(hipGraphExecDestroy(p->gen_graph));
-        p->step_graph = p->loop_graph = p->gen_graph = nullptr;
+        p->step_graph = p->gen_graph = nullptr;
         p->kv = kv;
     }
     return Q_OK;
@@ -716,7 +708,8 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
     const size_t o_pm = carve((size_t)cfg.n_heads * nch * 4), o_ps = carve((size_t)cfg.n_heads * nch * 4);
     const size_t o_op = carve(nch * cfg.n_heads * hd * 4);
     const size_t o_ct = carve(tab * 4), o_st = carve(tab * 4);
-    const size_t o_tok = carve(4), o_pos = carve(4), o_hn = carve(4), o_hist = carve((size_t)p->hist_cap * 4);
+    const size_t o_tok = carve(4), o_pos = carve(4), o_lp = carve(4), o_hn = carve(4);
+    const size_t o_hist = carve((size_t)p->hist_cap * 4);
     const size_t o_aw = carve(argmax_workspace_bytes(cfg.vocab_size));
     const size_t o_ap = carve((size_t)2 * kGemvAmaxMaxParts * 4);
     hipError_t e = hipMalloc(&p->arena, bytes);
@@ -730,6 +723,8 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
         plan_destroy(st);
         return Q_ERR_ALLOC_FAILED;
     }
+    p->pinned[2] = 0;  // (sources of small copies)
+    p->pinned[3] = 1;
     p->arena_bytes = bytes;
     uint8_t* A = p->arena;
     p->x = reinterpret_cast<float*>(A + o_x);
@@ -749,6 +744,7 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
     p->sin_tab = reinterpret_cast<float*>(A + o_st);
     p->tok = reinterpret_cast<uint32_t*>(A + o_tok);
     p->pos = reinterpret_cast<uint32_t*>(A + o_pos);
+    p->looped = reinterpret_cast<uint32_t*>(A + o_lp);
     p->hist_n = reinterpret_cast<uint32_t*>(A + o_hn);
     p->hist = reinterpret_cast<uint32_t*>(A + o_hist);
     p->amax_ws = reinterpret_cast<float*>(A + o_aw);
@@ -820,11 +816,15 @@ q_error_code llama_forward(q_llama_model* __restrict__ model, q_context* __restr
     QH_TRY_CODE(check_kv(p, ctx));
     QH_TRY_CODE(bind_kv(p, ctx));
     if (seq_len == 1) {
-        if (!p->step_graph) QH_TRY_CODE(capture(p, Feed::host, &p->step_graph));
+        if (!p->step_graph) QH_TRY_CODE(capture(p, false, &p->step_graph));
         QH_TRY(hipStreamSynchronize(p->stream));  // pinned staging is reused each step
         p->pinned[0] = tokens[0];
         p->pinned[1] = pos;
         // (the step's embedding launch reads them from there)
+        if (p->loop_set) {
+            QH_TRY(hipMemcpyAsync(p->looped, &p->pinned[2], 4, hipMemcpyHostToDevice, p->stream));
+            p->loop_set = false;
+        }
         QH_TRY(hipGraphLaunch(p->step_graph, p->stream));
     } else {
         QH_TRY_CODE(prefill_alloc(p));
@@ -905,11 +905,10 @@ q_error_code qh_llama_generate(q_llama_model* model, q_context* ctx, uint32_t to
     if (!p) return Q_ERR_INVALID_ARG;
     QH_TRY_CODE(check_kv(p, ctx));
     QH_TRY_CODE(bind_kv(p, ctx));
-    if (!p->gen_graph) QH_TRY_CODE(capture(p, Feed::greedy, &p->gen_graph));
+    if (!p->gen_graph) QH_TRY_CODE(capture(p, true, &p->gen_graph));
     QH_TRY(hipStreamSynchronize(p->stream));
     p->pinned[0] = token;
     p->pinned[1] = pos;
-    p->pinned[2] = 0;
     QH_TRY(hipMemcpyAsync(p->tok, &p->pinned[0], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->pos, &p->pinned[1], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->hist_n, &p->pinned[2], 4, hipMemcpyHostToDevice, p->stream));
@@ -952,7 +951,7 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     if (!p) return Q_ERR_INVALID_ARG;
     QH_TRY_CODE(check_kv(p, ctx));
     QH_TRY_CODE(bind_kv(p, ctx));
-    if (!p->loop_graph) QH_TRY_CODE(capture(p, Feed::loop, &p->loop_graph));
+    if (!p->step_graph) QH_TRY_CODE(capture(p, false, &p->step_graph));
     const uint32_t V = p->cfg.vocab_size;
     if (!p->sample_ws) {
         const size_t wb = sample_workspace_bytes(V);
@@ -969,7 +968,8 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     QH_TRY(hipStreamSynchronize(p->stream));
     p->pinned[0] = token;
     p->pinned[1] = pos;
-    p->pinned[2] = 0;
+    QH_TRY(hipMemcpyAsync(p->looped, &p->pinned[3], 4, hipMemcpyHostToDevice, p->stream));
+    p->loop_set = true;
     QH_TRY(hipMemcpyAsync(p->tok, &p->pinned[0], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->pos, &p->pinned[1], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->hist_n, &p->pinned[2], 4, hipMemcpyHostToDevice, p->stream));
@@ -978,7 +978,7 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     QH_TRY(hipEventCreate(&e1));
     QH_TRY(hipEventRecord(e0, p->stream));
     for (uint32_t i = 0; i < n_steps; ++i) {
-        QH_TRY(hipGraphLaunch(p->loop_graph, p->stream));
+        QH_TRY(hipGraphLaunch(p->step_graph, p->stream));
         sp.r = sample_draw();
         QH_TRY(launch_sample(p->logits, sp, p->sample_ws, p->tok, p->stream));
         QH_TRY(launch_token_feedback(p->tok, p->pos, p->hist, p->hist_n, p->hist_cap, p->stream));
