@@ -280,6 +280,27 @@ def test_generate_sampled_matches_host_loop(qa, tmp_path):
         m.close()
 
 
+@pytest.mark.parametrize("vocab", [301, 302, 303, 1, 3])
+def test_forward_odd_vocabularies(qa, tmp_path, vocab):
+    """The logits leave the device four at a time: vocabularies that end in a
+    part of four (or are one), one token and a prompt, every logit against
+    the oracle."""
+    h = qa.QorusHeader(vocab=vocab, dim=256, hidden=512, n_layers=1, n_heads=2, n_kv=1, max_seq=64)
+    P = 9
+    m, blob, kv = build(qa, tmp_path, h, 47, P)
+    try:
+        ref = orc.DecodeOracle(blob, kv.copy())
+        toks = [int(t) for t in orc.rng_for(47, vocab).integers(0, vocab, 6)]
+        _, lg_ref = ref.step(toks[0], P)
+        assert rel_err(m.forward(toks[:1], P), lg_ref) <= 1e-4
+        for i, t in enumerate(toks[1:-1]):
+            ref.fill(t, P + 1 + i)
+        _, lg_ref = ref.step(toks[-1], P + 5)
+        assert rel_err(m.forward(toks[1:], P + 1), lg_ref) <= 1e-4
+    finally:
+        m.close()
+
+
 def _q4_rows(blob, lay, name, rows, cols):
     """Writable [rows, cols/32, 20] view of a Q4_0 matrix inside a model blob."""
     off = lay[name]
