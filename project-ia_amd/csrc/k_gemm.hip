@@ -25,11 +25,12 @@
 //    gives NaN outputs (the GEMV kernel's convention).
 //
 // Tiling: past 64 tokens k_gemm_q4_p (below), 256 (or 192) rows x 128 tokens
-// a workgroup; 33 to 64 tokens k_gemm_q4, 256 rows x 64 tokens.  K advances in
-// steps of 2 blocks staged in LDS; the weights stay raw nibble blocks + scales
-// there and are dequantized per lane right before the MFMA.  Up to 32 tokens
-// k_gemm_q4_s, 64 (or 32) rows, everything straight to registers.  Workgroups are ordered so that each XCD keeps one token tile of X
-// resident in its L2 and streams the weight rows.
+// a workgroup, its workgroups ordered so that each XCD keeps one token tile of
+// X resident in its L2 and streams the weight rows; 33 to 64 tokens k_gemm_q4,
+// 256 rows x 64 tokens.  K advances in steps of 2 blocks staged in LDS; the
+// weights stay raw nibble blocks + scales there and are dequantized per lane
+// right before the MFMA.  Up to 32 tokens k_gemm_q4_s, 64 (or 32) rows,
+// everything straight to registers.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -326,7 +327,7 @@ __device__ __forceinline__ h8v unpack8(uint32_t w) {
     return h8v{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
-// The kernel of 33 to 64 tokens.  X hi/lo rows (padded: conflict-free 16-byte
+// The kernel of 33 to 64 tokens (one 64-token tile).  X hi/lo rows (padded: conflict-free 16-byte
 // reads) and the weight blocks go through registers into double-buffered LDS,
 // one barrier per K-step; global loads run ahead of the LDS stages, X one step
 // (L2 hits), the weight blocks two (HBM latency).
@@ -335,18 +336,16 @@ __device__ __forceinline__ h8v unpack8(uint32_t w) {
 constexpr int kGemmWM = 4;  // waves, one below the other
 
 __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
-    constexpr int WM = kGemmWM, WT = 1, MI = 4, JT = 4, KB = kKB;
-    constexpr int NT = 64 * WM * WT;
+    constexpr int MI = 4, JT = 4, KB = kKB;
+    constexpr int NT = 64 * kGemmWM;
     constexpr int WR = 16 * MI;  // weight rows per wave
-    constexpr int BM = WR * WM;
-    constexpr int BT = 16 * JT * WT;
+    constexpr int BM = WR * kGemmWM;
+    constexpr int BT = 16 * JT;
     constexpr int XCK = 4 * KB;                       // 16-byte X chunks per staged row and part
     constexpr int XROW = 32 * KB + 8;                 // LDS halfs per staged X row (8 pad)
     constexpr int XCH = 2 * XCK * BT / NT;            // 16-byte X chunks per thread per K-step
-    constexpr int WBL = (BM * KB + NT - 1) / NT;      // weight blocks per thread per K-step
-    constexpr bool kWAll = WBL * NT == BM * KB;       // every thread stages WBL blocks
-    static_assert(XCH * NT == 2 * XCK * BT, "tile/thread mismatch");
-    static_assert(BM * KB % 64 == 0, "weight staging threads come in whole waves");
+    constexpr int WBL = BM * KB / NT;                 // weight blocks per thread per K-step
+    static_assert(XCH * NT == 2 * XCK * BT && WBL * NT == BM * KB, "tile/thread mismatch");
     static_assert(KB == 2, "K-step of 2 blocks");
     static_assert(kInner % KB == 0, "inner sums end on K-step boundaries");
     // A row's blocks sit in its KB slots rotated by the row, so that the
@@ -357,25 +356,12 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
     __shared__ __attribute__((aligned(16))) uint32_t lw[2][BM][KB][4];
     __shared__ __attribute__((aligned(16))) float ls[2][KB][BM];
 
-    // ---- tile of this workgroup ----
-    const uint32_t n_mt = a.mt_end[a.nseg - 1] * a.split;  // (m-tile, split) pairs
-    uint32_t mm, tt;
-    {
-        const uint32_t b = blockIdx.x;
-        if (a.xcd_map) {
-            const uint32_t xcd = b & 7u, k = b >> 3;
-            tt = xcd % a.n_tt;
-            mm = xcd / a.n_tt + (8u / a.n_tt) * k;
-        } else {
-            tt = b % a.n_tt;
-            mm = b / a.n_tt;
-        }
-        if (mm >= n_mt) return;
-    }
+    // ---- tile of this workgroup: an (m-tile, split) pair ----
+    const uint32_t mm = blockIdx.x;
+    if (mm >= a.mt_end[a.nseg - 1] * a.split) return;
     const uint32_t mtile = mm / a.split, sp = mm % a.split;
     const uint32_t sg = seg_of_tile(a, mtile);
     const uint32_t m0 = (mtile - (sg ? a.mt_end[sg - 1] : 0u)) * BM;
-    const uint32_t t0 = tt * BT;
     const uint32_t M = a.M[sg];
     const uint32_t row_bytes = a.nblk * 20u;
     const uint32_t b_begin = sp * a.blk_per_split;
@@ -384,8 +370,7 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave % WM, wt = wave / WM;
+    const int wm = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     const __amdgpu_buffer_rsrc_t wrs =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.w[sg], 0, (int)(M * row_bytes), kBufFlagsG);
@@ -399,7 +384,7 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
     u4v gx[XCH];
     u4v gq[2][WBL];
     float gs[2][WBL];
-    // The thread's X chunks (row t0 + t, 8 halfs at column 8*ch of the step)
+    // The thread's X chunks (row t, 8 halfs at column 8*ch of the step)
     // as pointers fixed for the whole loop.
     const _Float16* xsrc[XCH];
 #pragma unroll
@@ -408,7 +393,7 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
         const uint32_t part = idx / (XCK * BT);
         const uint32_t rem = idx % (XCK * BT);
         const uint32_t t = rem / XCK, ch = rem % XCK;
-        xsrc[c] = (part ? a.xl : a.xh) + (size_t)(t0 + t) * a.N_pad + 8u * ch;
+        xsrc[c] = (part ? a.xl : a.xh) + (size_t)t * a.N_pad + 8u * ch;
     }
     auto load_x = [&](uint32_t step) {
         // < N_pad - (32 KB - 1): splits start on multiples of KB blocks and
@@ -425,8 +410,7 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
             const uint32_t idx = (uint32_t)(tid + NT * j);
             const uint32_t r = idx / KB, kb = idx % KB;
             const uint32_t b = b0 + kb;
-            // rows >= M read zeros; threads past the tile's blocks (kWAll
-            // false) load some row of the buffer and store nothing
+            // rows >= M read zeros
             const uint32_t off = (m0 + r) * row_bytes + b * 20u;
             // Blocks past the split's end are masked at the LDS store (a
             // select here would wait for the load right away).
@@ -450,11 +434,9 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
         for (int j = 0; j < WBL; ++j) {
             const uint32_t idx = (uint32_t)(tid + NT * j);
             const uint32_t r = idx / KB, kb = idx % KB;
-            if (kWAll || idx < (uint32_t)(BM * KB)) {  // wave-uniform: BM * KB is a multiple of 64
-                // A zero scale removes a masked block: its products are finite.
-                *reinterpret_cast<u4v*>(&lw[buf][r][kb ^ ((r >> kSwz) & (KB - 1u))][0]) = gq[buf][j];
-                ls[buf][kb][r] = b0 + kb < b_end ? gs[buf][j] : 0.0f;
-            }
+            // A zero scale removes a masked block: its products are finite.
+            *reinterpret_cast<u4v*>(&lw[buf][r][kb ^ ((r >> kSwz) & (KB - 1u))][0]) = gq[buf][j];
+            ls[buf][kb][r] = b0 + kb < b_end ? gs[buf][j] : 0.0f;
         }
     };
     using I0 = std::integral_constant<int, 0>;
@@ -505,7 +487,7 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
             // weight subtiles.
 #pragma unroll
             for (int j = 0; j < JT; ++j) {
-                const int t = 16 * JT * wt + 16 * j + lr;
+                const int t = 16 * j + lr;
                 const h8v Ah = *reinterpret_cast<const h8v*>(&lx[buf][0][t][32 * kb + 8 * lq]);
                 const h8v Al = *reinterpret_cast<const h8v*>(&lx[buf][1][t][32 * kb + 8 * lq]);
 #pragma unroll
@@ -542,7 +524,7 @@ __global__ __launch_bounds__(64 * kGemmWM) void k_gemm_q4(const GemmArgs a) {
         const uint32_t m = m0 + WR * wm + 16 * i + 4 * lq;
 #pragma unroll
         for (int j = 0; j < JT; ++j) {
-            const uint32_t t = t0 + 16 * JT * wt + 16 * j + lr;
+            const uint32_t t = 16 * j + lr;
             const f4v v = outer[i][j] + inner[i][j];
             if (m < M && t < a.T) {
                 if (a.split > 1) {
