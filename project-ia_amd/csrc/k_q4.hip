@@ -828,14 +828,14 @@ __global__ __launch_bounds__(64 * W * G) void k_gemv_p(const GemvArgs a) {
     }
 }
 
-// W waves split K, G independent row groups per workgroup, RW rows per wave
-// (processed R at a time, the next batch loaded while the current one is
+// Inputs past the persistent kernel's width: W waves split K, RW rows per
+// workgroup (processed R at a time, the next batch loaded while the current one is
 // computed), J block columns per lane per K-chunk (K-chunk = 64*W*J blocks).
 // Every load is unconditional: out-of-range rows/columns read a clamped,
 // in-bounds address and are masked (scale and digits zeroed), so the
 // compiler keeps all loads of a batch in flight together.
-template <int W, int J, int G, int RW, int R>
-__global__ __launch_bounds__(64 * W * G) void k_gemv(const GemvArgs a) {
+template <int W, int J, int RW, int R>
+__global__ __launch_bounds__(64 * W) void k_gemv(const GemvArgs a) {
     constexpr int kChunk = 64 * W * J;
     constexpr int NB = RW / R;
     static_assert(RW % R == 0, "RW must be a multiple of R");
@@ -854,10 +854,8 @@ __global__ __launch_bounds__(64 * W * G) void k_gemv(const GemvArgs a) {
     const uint32_t M = a.M[sg];
 
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int kw = wave % W;
-    const int g = wave / W;
-    const uint32_t row0 = (t - tbase) * (G * RW) + g * RW;
+    const int kw = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t row0 = (t - tbase) * RW;
     const size_t row_bytes = (size_t)a.nblk * 20u;
 
     float acc[RW];
@@ -959,55 +957,26 @@ __global__ __launch_bounds__(64 * W * G) void k_gemv(const GemvArgs a) {
     wave_row_totals<RW>(acc);
     float* __restrict__ y = a.y[sg];
     const float* __restrict__ res = a.res[sg];
-    if constexpr (W == 1) {
-        if (lane < RW) {
-            float v = acc[0], pv = acc[1];
+    __shared__ float red[W][RW];
+    if (lane == 0) {
 #pragma unroll
-            for (int r = 1; r < RW; ++r) v = (r == lane) ? acc[r] : v;
+        for (int r = 0; r < RW; ++r) red[kw][r] = acc[r];
+    }
+    __syncthreads();
+    const int r = threadIdx.x;
+    if (r < RW) {
+        float v = red[0][r];
 #pragma unroll
-            for (int r = 0; r < RW; ++r) pv = (r == (lane ^ 1)) ? acc[r] : pv;
-            const uint32_t row = row0 + lane;
-            const uint32_t hd = a.hd[sg];
-            float* dst = y + row;
-            if (hd) {
-                const uint32_t pos = *a.pos;
-                const uint32_t i = row % hd;
-                if ((a.rope_mask >> sg) & 1u) {
-                    // Pair (x0, x1) = (row&~1, row|1): y0 = x0*c - x1*s,
-                    // y1 = x1*c + x0*s, products rounded separately.
-                    const float c = a.cos_tab[(size_t)pos * hd + i];
-                    const float sn = a.sin_tab[(size_t)pos * hd + i];
-                    const float t0 = v * c, t1 = pv * sn;
-                    v = (lane & 1) ? t0 + t1 : t0 - t1;
-                }
-                dst = y + (size_t)pos * a.pos_stride[sg] + (size_t)(row / hd) * a.head_stride[sg] + i;
-            }
-            if (row < M) *dst = res ? res[row] + v : v;
-        }
-    } else {
-        __shared__ float red[G][W][RW];
-        if (lane == 0) {
-#pragma unroll
-            for (int r = 0; r < RW; ++r) red[g][kw][r] = acc[r];
-        }
-        __syncthreads();
-        const int tid = threadIdx.x;
-        if (tid < G * RW) {
-            const int gg = tid / RW, r = tid % RW;
-            float v = red[gg][0][r];
-#pragma unroll
-            for (int k2 = 1; k2 < W; ++k2) v += red[gg][k2][r];
-            const uint32_t row = (t - tbase) * (G * RW) + gg * RW + r;
-            if (row < M) y[row] = res ? res[row] + v : v;
-        }
+        for (int k2 = 1; k2 < W; ++k2) v += red[k2][r];
+        const uint32_t row = row0 + r;
+        if (row < M) y[row] = res ? res[row] + v : v;
     }
 }
 
-template <int W, int J, int G, int RW, int R>
+template <int W, int J, int RW, int R>
 static hipError_t run_gemv(const GemvSeg* segs, int nseg, uint32_t nblk, const uint4* xd, hipStream_t s,
                            const GemvDecode* dec) {
     GemvArgs a{};
-    constexpr uint32_t tile_rows = G * RW;
     uint32_t tiles = 0;
     for (int i = 0; i < 4; ++i) {
         if (i < nseg) {
@@ -1015,15 +984,8 @@ static hipError_t run_gemv(const GemvSeg* segs, int nseg, uint32_t nblk, const u
             a.y[i] = segs[i].y;
             a.res[i] = segs[i].res;
             a.M[i] = segs[i].M;
-            a.hd[i] = segs[i].hd;
-            a.head_stride[i] = segs[i].head_stride;
-            a.pos_stride[i] = segs[i].pos_stride;
-            if (segs[i].rope) a.rope_mask |= 1u << i;
-            // The decode epilogue exists on the single-wave-per-row path only,
-            // and RoPE needs whole pairs inside one wave's rows.
-            if (segs[i].hd && (W != 1 || !dec || !dec->pos || (segs[i].hd % 2) != 0)) return hipErrorInvalidValue;
-            if (segs[i].rope && (!dec->cos_tab || !dec->sin_tab || (RW % 2) != 0)) return hipErrorInvalidValue;
-            tiles += (segs[i].M + tile_rows - 1) / tile_rows;
+            if (segs[i].hd || segs[i].rope) return hipErrorInvalidValue;  // decode epilogue: persistent kernel only
+            tiles += (segs[i].M + RW - 1) / RW;
         }
         a.tile_end[i] = tiles;
     }
@@ -1031,14 +993,9 @@ static hipError_t run_gemv(const GemvSeg* segs, int nseg, uint32_t nblk, const u
     a.nblk = nblk;
     a.pad = xd_pad(nblk);
     a.xd = xd;
-    if (dec) {
-        a.pos = dec->pos;
-        a.cos_tab = dec->cos_tab;
-        a.sin_tab = dec->sin_tab;
-        if (dec->in_part) return hipErrorInvalidValue;  // norm scale: persistent kernel only
-    }
+    if (dec && dec->in_part) return hipErrorInvalidValue;  // norm scale: persistent kernel only
     if (tiles == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_gemv<W, J, G, RW, R>), dim3(tiles), dim3(64 * W * G), 0, s, a);
+    hipLaunchKernelGGL((k_gemv<W, J, RW, R>), dim3(tiles), dim3(64 * W), 0, s, a);
     return hipGetLastError();
 }
 
@@ -1179,7 +1136,7 @@ hipError_t launch_gemv(const GemvSeg* segs, int nseg, uint32_t nblk, const uint4
                        const GemvDecode* dec) {
     if (nseg < 1 || nseg > 4) return hipErrorInvalidValue;
     if (nblk <= kGemvPMaxBlk) return run_gemv_shape(segs, nseg, nblk, xd, (const float*)nullptr, s, dec);
-    return run_gemv<8, 2, 1, 16, 4>(segs, nseg, nblk, xd, s, dec);
+    return run_gemv<8, 2, 16, 4>(segs, nseg, nblk, xd, s, dec);
 }
 
 // h = silu(W_gate . n) * (W_up . n), n = RMSNorm(x) with weight norm_w (the
@@ -1217,7 +1174,7 @@ hipError_t launch_gemv_f32(const GemvSeg* segs, int nseg, uint32_t N, const floa
     if (!ws || (dec && dec->norm_w)) return hipErrorInvalidValue;
     hipError_t e = launch_xprep(x, N, nullptr, 0.0f, nullptr, ws, s);
     if (e != hipSuccess) return e;
-    return run_gemv<8, 2, 1, 16, 4>(segs, nseg, nblk, ws, s, dec);
+    return run_gemv<8, 2, 16, 4>(segs, nseg, nblk, ws, s, dec);
 }
 
 // LM-head form of launch_gemv_f32 (one segment, plain store, 2048 < N <=
