@@ -58,7 +58,7 @@ using namespace qh;
 extern "C" q_error_code qh_gemv_q4_f32_softmax_argmax_noalloc(const q_tensor* W, const float* x, float* logits,
                                                               float* probs, uint32_t* index_out, qh_stream s) {
     QH_TRY_CODE(validate_gemv_softmax(W, x, logits, probs, index_out, false, nullptr));
-    if (W->ne[1] / 32 > kGemvF32MaxBlk)
+    if (W->ne[1] > 16384)  // the entry point's documented limit
         return fail_code(Q_ERR_INVALID_SIZE,
                          "qh_gemv_q4_f32_softmax_argmax_noalloc: N above 16384");
     if (gemv_softmax_ws_bytes(W->ne[0]) > kScratchBytes)

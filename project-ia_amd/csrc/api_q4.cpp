@@ -54,8 +54,8 @@ static q_error_code gemv_device(const q_tensor* W, const void* wdev, const float
     return Q_OK;
 }
 
-// Callers of wider inputs bring a workspace (or take the library's); the
-// launch touches it past the width of the in-kernel conversion.
+// Callers of inputs wider than the in-kernel conversion bring a workspace (or
+// take the library's).
 static bool needs_workspace(uint32_t N) { return N / 32 > kGemvF32MaxBlk; }
 
 }  // namespace qh

@@ -1128,14 +1128,13 @@ static hipError_t run_gemv_shape(const GemvSeg* segs, int nseg, uint32_t nblk, A
     if (nblk <= 896) return run_gemv_p<14, 1, 1, 2>(segs, nseg, nblk, args...);
     return run_gemv_p<16, 1, 1, 2>(segs, nseg, nblk, args...);
 }
-constexpr uint32_t kGemvPMaxBlk = 1024;
 
 // Prepared digits; inputs past the persistent kernel's width run the
 // tile-per-workgroup one.
 hipError_t launch_gemv(const GemvSeg* segs, int nseg, uint32_t nblk, const uint4* xd, hipStream_t s,
                        const GemvDecode* dec) {
     if (nseg < 1 || nseg > 4) return hipErrorInvalidValue;
-    if (nblk <= kGemvPMaxBlk) return run_gemv_shape(segs, nseg, nblk, xd, (const float*)nullptr, s, dec);
+    if (nblk <= kGemvF32MaxBlk) return run_gemv_shape(segs, nseg, nblk, xd, (const float*)nullptr, s, dec);
     return run_gemv<8, 2, 16, 4>(segs, nseg, nblk, xd, s, dec);
 }
 
@@ -1163,14 +1162,14 @@ hipError_t launch_gemv_swiglu(const uint8_t* w_gate, const uint8_t* w_up, uint32
     return launch_gemv_p<1, 2, 4, kRT, true, true>(a, tiles, s);
 }
 
-// fp32 input: inputs of up to kGemvPMaxBlk blocks are converted inside the
+// fp32 input: inputs of up to kGemvF32MaxBlk blocks are converted inside the
 // GEMV (one launch); wider ones go through k_xprep into ws first.
 hipError_t launch_gemv_f32(const GemvSeg* segs, int nseg, uint32_t N, const float* x, uint4* ws, hipStream_t s,
                            const GemvDecode* dec) {
     if (nseg < 1 || nseg > 4 || N == 0 || N % 32 != 0) return hipErrorInvalidValue;
     if (dec && dec->in_part) return hipErrorInvalidValue;
     const uint32_t nblk = N / 32;
-    if (nblk <= kGemvPMaxBlk) return run_gemv_shape(segs, nseg, nblk, (const uint4*)nullptr, x, s, dec);
+    if (nblk <= kGemvF32MaxBlk) return run_gemv_shape(segs, nseg, nblk, (const uint4*)nullptr, x, s, dec);
     if (!ws || (dec && dec->norm_w)) return hipErrorInvalidValue;
     hipError_t e = launch_xprep(x, N, nullptr, 0.0f, nullptr, ws, s);
     if (e != hipSuccess) return e;

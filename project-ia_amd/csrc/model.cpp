@@ -556,7 +556,7 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
     // This build: version-3 layout, GQA group dividing the heads, 128-wide
     // heads, d_model up to 16384 (the Q|K|V epilogue's persistent GEMV).
     if (h->version < 3 || h->hidden_dim == 0 || h->max_seq_len == 0) return Q_ERR_INVALID_CONFIG;
-    if (h->dim / 32 > kGemvF32MaxBlk) return Q_ERR_INVALID_CONFIG;
+    if (h->dim > 16384) return Q_ERR_INVALID_CONFIG;
     if (h->hidden_dim > 32768) return Q_ERR_INVALID_CONFIG;  // the prefill GEMM converts rows of N <= 32768
     const uint32_t group = h->n_kv_heads ? h->n_heads / h->n_kv_heads : 0;
     if (group != 1 && group != 2 && group != 4 && group != 8) return Q_ERR_INVALID_CONFIG;  // GQA groups built
@@ -749,7 +749,9 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
     p->hist = reinterpret_cast<uint32_t*>(A + o_hist);
     p->amax_ws = reinterpret_cast<float*>(A + o_aw);
     p->amax_parts = reinterpret_cast<float*>(A + o_ap);
-    p->fused = cfg.dim / 32 <= 128 && cfg.hidden_dim / 32 <= kGemvF32MaxBlk && (p->kvd % 32) == 0;
+    // (the fused layer's prologues hold a d_model of 4096; the FFN widths are
+    // those it was measured and tested with)
+    p->fused = cfg.dim <= 4096 && cfg.hidden_dim <= 16384 && (p->kvd % 32) == 0;
     st->plan = p;
     st->dev_arena = p->arena;
     st->dev_arena_size = bytes;

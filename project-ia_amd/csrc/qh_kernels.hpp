@@ -64,11 +64,11 @@ struct GemvDecode {
 // y = W . x for up to 4 segments sharing the same x (digit planes xd).
 hipError_t launch_gemv(const GemvSeg* segs, int nseg, uint32_t nblk, const uint4* xd,
                        hipStream_t s, const GemvDecode* dec = nullptr);
-// Same from the fp32 input x[N]: inputs of up to 1024 32-element blocks are
-// converted to digit planes inside the GEMV launch; wider ones are prepared
-// into ws (xd_bytes(N/32) bytes) by a separate launch first.  Entry points
-// ask for a workspace past kGemvF32MaxBlk blocks.
-constexpr uint32_t kGemvF32MaxBlk = 512;
+// Same from the fp32 input x[N]: inputs of up to kGemvF32MaxBlk 32-element
+// blocks are converted to digit planes inside the GEMV launch (the widths of
+// its launch shapes); wider ones are prepared into ws (xd_bytes(N/32) bytes)
+// by a separate launch first.
+constexpr uint32_t kGemvF32MaxBlk = 1024;
 // h[M] = silu(W_gate . n) * (W_up . n) with n = RMSNorm(x, norm_w, eps) made
 // in the GEMV's prologue (x fp32, N <= 4096): the decode step's FFN input.
 hipError_t launch_gemv_swiglu(const uint8_t* w_gate, const uint8_t* w_up, uint32_t M, uint32_t N, const float* x,
