@@ -50,6 +50,12 @@
 
 namespace qh {
 
+// Raw buffer resource word 3 for gfx9-family parts (32-bit untyped data, no
+// swizzle); out-of-range reads return zero, out-of-range stores
+// are dropped.
+constexpr int kBufFlags = 0x00020000;
+typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
+
 // ---------------------------------------------------------------------------
 // Dequantization: reference src/ops/avx2/dequantize.c:25-72.
 // off = -8*s; out[e] = fma((float)q_e, s, off); element e in byte e>>1,
@@ -59,18 +65,19 @@ namespace qh {
 // consecutive blocks: 5 coalesced dword loads per lane, a turn through LDS,
 // and 8 rounds of 16-byte stores, each round 1 KB of consecutive output.
 // (With a block per thread, a wave's store instruction touched 64 cache
-// lines 16 bytes at a time: 1,835,008 blocks took 90.1 us = 3.0 TB/s; this
-// form takes 49.5 us = 5.5 TB/s.)  NT: the stores carry the non-temporal
-// hint, 40.4 us = 6.7 TB/s at that size.
+// lines 16 bytes at a time: 1,835,008 blocks took 90.1 us = 3.0 TB/s; in this
+// form plain stores take 42.3, the ones below 40.2 = 6.8 TB/s.)
+// kPolicy: cache policy of the stores (see kDequantNtBlocks).
 // ---------------------------------------------------------------------------
-typedef float f4_nt __attribute__((ext_vector_type(4)));
+constexpr int kStoreNt = 2, kStoreSc1 = 16;  // policy bits: non-temporal, write through the L2
 
-template <bool NT>
+template <int kPolicy>
 __global__ __launch_bounds__(256) void k_dequant(const uint32_t* __restrict__ blocks, float* __restrict__ out,
                                                  uint64_t n_blocks) {
     constexpr uint32_t kDw = 5;  // dwords of a block: 16 nibble bytes, the scale
     __shared__ uint32_t lds[4][64 * kDw];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint64_t b0 = ((uint64_t)blockIdx.x * 4u + wave) * 64u;  // the wave's first block
     if (b0 >= n_blocks) return;                                    // no workgroup barrier follows
     const uint32_t nb = (uint32_t)(n_blocks - b0 < 64u ? n_blocks - b0 : 64u);
@@ -86,38 +93,45 @@ __global__ __launch_bounds__(256) void k_dequant(const uint32_t* __restrict__ bl
     // (a wave's LDS writes complete before its later reads; the fence keeps
     // the compiler from moving those up)
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    f4_nt* o = reinterpret_cast<f4_nt*>(out + b0 * 32u);
+    // the wave's output; stores past its last block are dropped
+    const __amdgpu_buffer_rsrc_t ro =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(out + b0 * 32u), 0, (int)(nb * 128u), kBufFlags);
 #pragma unroll
     for (uint32_t i = 0; i < 8; ++i) {
         const uint32_t g = i * 64u + lane, b = g >> 3, c = g & 7u;  // elements 4c .. 4c+3 of block b
         const uint32_t w = lds[wave][b * kDw + (c >> 1)] >> (16u * (c & 1u));
         const float s = __uint_as_float(lds[wave][b * kDw + 4u]);
         const float off = -8.0f * s;
-        f4_nt r;
+        v4u32 r;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = fmaf((float)((w >> (4 * j)) & 15u), s, off);
-        if (b < nb) {
-            if constexpr (NT)
-                __builtin_nontemporal_store(r, o + g);
-            else
-                o[g] = r;
-        }
+        for (int j = 0; j < 4; ++j) r[j] = __float_as_uint(fmaf((float)((w >> (4 * j)) & 15u), s, off));
+        __builtin_amdgcn_raw_buffer_store_b128(r, ro, g * 16u, 0, kPolicy);
     }
 }
 
-// Outputs past the eight 4 MB L2 caches leave them before any reader comes,
-// so their stores carry the hint; smaller ones stay for the kernel that
-// reads them next (at 60,001 blocks, 7.7 MB, both take 6.5 us).
-constexpr uint64_t kDequantNtBlocks = (32ull << 20) / 128;
+// The stores write through the L2, which spares its write-backs: the data is
+// in the 256 MB memory-side cache when the kernel that reads it next comes.
+// Where blocks (20 bytes) and output (128) together pass that cache, they also
+// carry the non-temporal hint.  us alone / with a reading kernel behind / with
+// one that reads and writes:
+//   output   plain stores         write through        and non-temporal
+//     8 MB    3.4   13.1   12.3    3.5   12.6   12.1    3.4   12.9   13.1
+//    34 MB    8.2   28.2   28.2    7.0   28.1   27.4    7.3   30.7   33.2
+//    64 MB   12.6   31.1   43.2   10.5   30.8   42.6   11.5   33.7   52.8
+//   128 MB   23.8   49.8   81.4   19.6   49.4   78.9   22.6   53.8   96.3
+//   200 MB   35.7   73.6  159.7   31.7   72.8  157.6   34.8   83.0  160.6
+//   230 MB   45.5   99.7  187.3   43.5   96.5  186.0   39.4   91.8  184.7
+//   300 MB   66.2  152.2  240.0   63.5  150.5  238.1   53.5  134.8  239.9
+constexpr uint64_t kDequantNtBlocks = (256ull << 20) / (20 + 128);
 
 hipError_t launch_dequant(const uint8_t* blocks, float* out, uint64_t n_blocks, hipStream_t s) {
     if (n_blocks == 0) return hipSuccess;
     const uint64_t grid = (n_blocks + 255) / 256;
     const uint32_t* b = reinterpret_cast<const uint32_t*>(blocks);
     if (n_blocks > kDequantNtBlocks)
-        hipLaunchKernelGGL(k_dequant<true>, dim3((uint32_t)grid), dim3(256), 0, s, b, out, n_blocks);
+        hipLaunchKernelGGL((k_dequant<kStoreSc1 | kStoreNt>), dim3((uint32_t)grid), dim3(256), 0, s, b, out, n_blocks);
     else
-        hipLaunchKernelGGL(k_dequant<false>, dim3((uint32_t)grid), dim3(256), 0, s, b, out, n_blocks);
+        hipLaunchKernelGGL((k_dequant<kStoreSc1>), dim3((uint32_t)grid), dim3(256), 0, s, b, out, n_blocks);
     return hipGetLastError();
 }
 
@@ -240,11 +254,6 @@ __device__ __forceinline__ float gemv_norm_scale(const float* __restrict__ part,
     const float r0 = __builtin_amdgcn_rsqf(av);
     return (r0 * (3.0f - av * (r0 * r0))) * 0.5f;
 }
-
-// Raw buffer resource word 3 for gfx9-family parts (32-bit untyped data, no
-// swizzle); out-of-range reads return zero.
-constexpr int kBufFlags = 0x00020000;
-typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 
 // Store one finished row (value v, RoPE partner pv) of segment sg, with the
 // residual rv and the RoPE cos/sin (c, sn) of the row already loaded.  RoPE
