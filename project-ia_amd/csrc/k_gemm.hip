@@ -284,7 +284,10 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& a, uint32_t sg, uint3
 }
 
 // gemm_store of rows m .. m+3 (those below the segment's M), with 16-byte
-// accesses where the row length keeps them aligned.
+// accesses where the row length is a multiple of 4.  They are 4-byte aligned:
+// so is Y, and a second launch's piece of a segment can start at any row.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
 __device__ __forceinline__ void gemm_store4(const GemmArgs& a, uint32_t sg, uint32_t t, uint32_t m, f4v v) {
     const uint32_t M = a.M[sg];
     if ((a.ld[sg] & 3u) != 0 || m + 3 >= M) {
@@ -296,9 +299,9 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs& a, uint32_t sg, uint
     const float2 mt = a.meta[t];
     const size_t i = (size_t)t * a.ld[sg] + m;
     f4v y = v * mt.x;
-    if (a.res[sg]) y = *reinterpret_cast<const f4v*>(a.res[sg] + i) + y;
+    if (a.res[sg]) y = *reinterpret_cast<const f4u*>(a.res[sg] + i) + y;
     if (mt.y != 0.0f) y = f4v{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
-    *reinterpret_cast<f4v*>(a.y[sg] + i) = y;
+    *reinterpret_cast<f4u*>(a.y[sg] + i) = y;
 }
 
 // (a & mask) | c in one instruction (the compiler splits it in two when both

@@ -190,6 +190,27 @@ def test_gemm_two_tile_heights_match_single_launches(qa):
     check_rows(Ws[1], M, N, X, Ys[1], [0, 300, 511])
 
 
+def test_gemm_cut_inside_an_unaligned_segment(qa):
+    """The same with a first matrix of an odd row count: the second launch's
+    piece of the second matrix, whose row length allows 16-byte stores, starts
+    between 16-byte boundaries.  Outputs placed 4 bytes past one, too."""
+    Ms, N, T = [3955, 11956, 232], 1280, 1041
+    rng = orc.rng_for(43, 7)
+    Ws = [orc.gen_q4(M, N, rng) for M in Ms]
+    X = rng.standard_normal((T, N), dtype=np.float32)
+    Ys = Gemm(qa, Ws, Ms, N, T)(X)
+    for W, M, Y in zip(Ws, Ms, Ys):
+        (S,) = Gemm(qa, [W], [M], N, T)(X)
+        assert np.array_equal(Y, S), M
+    W, M, n = Ws[1][:256], 256, 70
+    g = Gemm(qa, [W], [M], N, n)
+    (S,) = g(X[:n])
+    buf = qa.DeviceBuffer(4 + n * M * 4)
+    qa.check(qa.lib().qh_gemm_q4_f32(g.t[0].addr, g.dX.ptr, n, buf.ptr + 4, g.ws.ptr, None))
+    qa.check(qa.lib().qh_device_synchronize())
+    assert np.array_equal(buf.download(np.float32, (n, M), 4), S)
+
+
 def test_gemm_scaled_and_nonfinite_rows(qa):
     """Per-token power-of-two scaling: rows of very different magnitude, an
     all-zero row, and a row holding Inf/NaN (-> NaN outputs for that token
