@@ -1080,10 +1080,14 @@ static uint32_t gemm_npad(uint32_t N) { return (N + 127u) & ~127u; }  // whole K
 // rows), the K split (partials plus a reduction pass when > 1; each split
 // keeps at least 32 blocks, and at most max_split), and, for whole-K
 // launches, a cut: rows from `cut` on (counted over the matrices laid end to
-// end) run in 192-row tiles in a second launch.  The cost model is measured
-// on MI355X at T = 2048: a launch takes rounds x (20 us + K-steps x 1.93 us
-// for 256-row tiles, 1.41 us for 192-row tiles), a round being up to 256
-// workgroups (one per CU); a reduction about 1 us plus its traffic at 5 TB/s.
+// end) run in 192-row tiles in a second launch.  The cost model: a launch takes
+// rounds x (20 us + K-steps x 1.93 us for 256-row tiles, 1.41 us for 192-row
+// tiles), a round being up to 256 workgroups (one per CU); a reduction about 1
+// us plus its traffic at 5 TB/s.  Its constants rank plans, they do not predict
+// a launch: one round alone takes 12 us + 2.07 a step and 10.6 + 1.70 (512 and
+// 2048 tokens, 16 to 64 steps; past those the clock falls), but plans made from
+// these figures differ for 1.5 % of shapes, and of 22 such ten were 2 to 6 %
+// slower (914|5709|1922 x 472 x 6592 167 -> 178 us) and two 1 % faster.
 // From 33 to 128 tokens (one 128-token tile) the plan instead takes the
 // smaller token tile of 64 or 128 holding them and the smallest K split (a
 // power of two, each split keeping kInner blocks) that gives at least 224
