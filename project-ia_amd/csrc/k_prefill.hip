@@ -1,6 +1,7 @@
 // k_prefill.hip -- batched-prefill kernels for gfx950 other than the GEMM:
 // token embedding rows, RoPE of the Q|K rows with the KV-cache stores, and
-// the causal attention of T queries over the cache on fp32 matrix cores.
+// the causal attention of T queries over the cache on fp16 matrix cores (every
+// fp32 operand in two fp16 parts, hi and lo).
 //
 // The prefill computes what T successive decode steps compute (reference
 // src/models/model.c:1655-1850 run with seq_len = 1 per token): token t at

@@ -279,15 +279,15 @@ __device__ __forceinline__ void prep_block_lo(const float (&v)[32], int k, uint4
     }
 }
 
-// prep_block split over the 4 lanes of an aligned lane quad: lane i of the
+// prep_block_hi split over the 4 lanes of an aligned lane quad: lane i of the
 // quad holds elements 8i..8i+7 of the block in v and gets dword i of every
 // level-1 plane (pl, already XORed with 0x88888888), the block's k and z
 // words, its level-1 maximum amax and maybe = maybe_wide (the cheap first
 // stage of the wide test).  The block maximum and magnitude sum are combined
 // across the quad, so all 4 lanes must call it together; the digits are
-// those of prep_block bit for bit.  quarter_wide completes the wide test
-// (the flag of prep_block), and prep_quarter_lo gives the same lane's dwords
-// of the level-2 planes of a wide block.  The second stage is kept apart so
+// those of prep_block_hi bit for bit.  quarter_wide completes the wide test
+// (prep_block_hi's flag), and prep_quarter_lo gives the same lane's dwords of
+// prep_block_lo's level-2 planes of a wide block.  The second stage is kept apart so
 // a caller converting several blocks per lane runs it once, after all of
 // them, and only when some lane of the wave needs it.
 __device__ __forceinline__ void prep_quarter(const float (&v)[8], uint32_t (&pl)[6], uint32_t& k_out,
