@@ -291,6 +291,14 @@ __device__ __forceinline__ void store_row_pre(const GemvArgs& a, uint32_t sg, ui
 // keep the default cache policy: the non-temporal hint made this kernel 4-10 %
 // slower (a block's 16-byte nibble load and its 4-byte scale load share
 // cache lines), although it speeds up plain one-pass 16-byte reads.
+//
+// Every instance begins on a 4 KB page: a decode step runs 4 of them of 11 to
+// 22 KB in turn, and each launch fetches its code anew over as few pages as it
+// can.  At 256-byte alignment the step's time moved with whatever lies ahead
+// of them in the file: two Llama-3-8B layers took 122.8 or 124.7 us by a
+// 256-byte shift (one fed token 133.9 or 135.8, a sampled one 398.4 or 400.3);
+// on pages 124.0 / 132.6 / 397.5 beside 125.0 / 136.4 / 400.4, at 1 KB
+// 125.5 / 134.6 / 399.8.
 // ---------------------------------------------------------------------------
 // SW: SwiGLU pair mode (W == 1): tile u holds rows i0..i0+RT/2-1 of w[0]
 // (W_gate) followed by the same rows of w[1] (W_up), i0 = u*RT/2, and stores
@@ -299,7 +307,7 @@ __device__ __forceinline__ void store_row_pre(const GemvArgs& a, uint32_t sg, ui
 // (largest value, first row holding it) of the rows it stored to a.amax, the
 // greedy argmax's partials (arg_better), so no separate pass re-reads y.
 template <int W, int J, int G, int RT, bool XF, bool SW = false, bool AM = false>
-__global__ __launch_bounds__(64 * W * G) void k_gemv_p(const GemvArgs a) {
+__global__ __launch_bounds__(64 * W * G) __attribute__((aligned(4096))) void k_gemv_p(const GemvArgs a) {
     static_assert(W == 1 || G == 1, "multi-wave K split runs one tile per workgroup");
     static_assert(!SW || (W == 1 && RT % 2 == 0), "SwiGLU pairs need one wave per group and even tiles");
     static_assert(!AM || (W == 1 && !SW), "argmax partials are taken in the one-wave store path");
