@@ -425,30 +425,32 @@ static_assert(bounded(0u, 1u) == 0u && bounded(2055u, 2056u) == 2055u && bounded
 // bounded here, ahead of every kernel that addresses by them (the position
 // steers the KV-cache stores): the host validates what it submits and the
 // device loops stay in range, so the bound only acts on a stray word.  They are
-// in device memory, or, with host and while *looped is 0, in two words of pinned
-// memory, and are then stored for the kernels behind: read once per workgroup,
-// as each read crosses the link.  A device loop over the same graph sets
-// *looped and stays off the link (a graph of its own for it took 2 MB of
-// device memory at the first loop).  With two 4-byte copies ahead of the step
+// in device memory, or, with host and unless its position word says otherwise,
+// in two words of pinned memory, and are then stored for the kernels behind:
+// one 8-byte read per workgroup, as each read crosses the link.  (For the loop
+// that keeps them on the device, a graph of its own took 2 MB of device memory
+// at its first call; a device word that says which holds, read ahead of the
+// pinned ones, gave that loop 0.7 us a token and cost every llama_forward 0.6,
+// 1 to 2 where nothing is cached.)  With two 4-byte copies ahead of the step
 // and one behind it for the logits, one layer of Llama-3-8B at position 2047
 // with an 8192-token vocabulary took 158 us from call to return; with the
 // reads and k_to_host 144 (150 with the words read by every thread).
 __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, uint32_t* tok, uint32_t* pos,
-                                               const uint32_t* host, const uint32_t* looped, uint32_t vocab,
-                                               uint32_t max_seq, uint32_t dim4, float4* __restrict__ x) {
+                                               const uint32_t* host, uint32_t vocab, uint32_t max_seq,
+                                               uint32_t dim4, float4* __restrict__ x) {
     __shared__ uint32_t t_s;
     if (threadIdx.x == 0) {
-        uint32_t t;
-        if (host && *looped == 0) {
-            const uint2 w = host_words(host);
-            t = w.x;
-            if (blockIdx.x == 0) {  // (no workgroup reads them here)
+        uint32_t p = blockIdx.x == 0 ? *pos : 0u;
+        uint2 w = make_uint2(0u, kOnDevice);
+        if (host) w = host_words(host);
+        const bool fed = w.y != kOnDevice;
+        const uint32_t t = fed ? w.x : *tok;
+        if (blockIdx.x == 0) {
+            if (fed) {  // (no other workgroup reads them here)
                 *tok = t;
-                *pos = bounded(w.y, max_seq);
+                p = w.y;
             }
-        } else {
-            t = *tok;
-            if (blockIdx.x == 0 && *pos >= max_seq) *pos = max_seq - 1u;
+            if (fed || p >= max_seq) *pos = bounded(p, max_seq);
         }
         t_s = bounded(t, vocab);
     }
@@ -458,12 +460,11 @@ __global__ __launch_bounds__(256) void k_embed(const float4* __restrict__ embd, 
         x[i] = embd[(size_t)t * dim4 + i];
 }
 
-hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host,
-                        const uint32_t* looped, uint32_t vocab, uint32_t max_seq, uint32_t dim, float* x,
-                        hipStream_t s) {
-    if (dim % 4 != 0 || vocab == 0 || max_seq == 0 || (host && !looped)) return hipErrorInvalidValue;
+hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host, uint32_t vocab,
+                        uint32_t max_seq, uint32_t dim, float* x, hipStream_t s) {
+    if (dim % 4 != 0 || vocab == 0 || max_seq == 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_embed, dim3((dim / 4 + 255) / 256), dim3(256), 0, s, reinterpret_cast<const float4*>(embd), tok,
-                       pos, host, looped, vocab, max_seq, dim / 4, reinterpret_cast<float4*>(x));
+                       pos, host, vocab, max_seq, dim / 4, reinterpret_cast<float4*>(x));
     return hipGetLastError();
 }
 

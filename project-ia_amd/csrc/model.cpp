@@ -58,7 +58,6 @@ struct ModelPlan {
     float *scores = nullptr, *part_max = nullptr, *part_sum = nullptr, *o_part = nullptr;
     float *cos_tab = nullptr, *sin_tab = nullptr;
     uint32_t *tok = nullptr, *pos = nullptr, *hist = nullptr, *hist_n = nullptr;
-    uint32_t* looped = nullptr;              // device: 1 while a loop keeps token/pos in device memory
     uint32_t hist_cap = 0;
     float* amax_ws = nullptr;                // multi-workgroup argmax partials
     float* amax_parts = nullptr;             // the LM-head GEMV's argmax partials
@@ -66,11 +65,10 @@ struct ModelPlan {
     float* kv = nullptr;
     size_t kv_layer_floats = 0;
     hipStream_t stream = nullptr;
-    hipGraphExec_t step_graph = nullptr;     // decode step, token/pos from the pinned words unless *looped
+    hipGraphExec_t step_graph = nullptr;     // decode step, token/pos from the pinned words, or on the device
     hipGraphExec_t gen_graph = nullptr;      // decode step + greedy feedback + pos advance
     void* sample_ws = nullptr;               // device workspace of sampled generation
-    uint32_t* pinned = nullptr;              // host staging: token, pos, 0, 1
-    bool loop_set = false;                   // *looped is 1 (since the last sampled generation)
+    uint32_t* pinned = nullptr;              // host staging: token, pos (or kOnDevice), 0, a loop's first pos
     float* pinned_logits = nullptr;          // host staging for the logits llama_forward returns
     // Batched prefill (llama_forward with seq_len > 1), allocated at its
     // first use: row buffers for pf_rows tokens and the GEMM workspace.
@@ -171,8 +169,8 @@ static hipError_t enqueue_step_fused(ModelPlan* p, bool feedback) {
         if (e != hipSuccess) return e;   \
     } while (0)
     const uint32_t nblk_d = c.dim / 32;
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, p->looped, c.vocab_size,
-                      c.max_seq_len, c.dim, p->x, s));
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, c.vocab_size, c.max_seq_len,
+                      c.dim, p->x, s));
     for (uint32_t l = 0; l < c.n_layers; ++l) {
         const LayerDev& L = p->layers[l];
         float* kvl = p->kv + (size_t)l * p->kv_layer_floats;
@@ -261,8 +259,8 @@ static hipError_t enqueue_step(ModelPlan* p, bool feedback) {
         e = (x);                         \
         if (e != hipSuccess) return e;   \
     } while (0)
-    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, p->looped, c.vocab_size,
-                      c.max_seq_len, c.dim, p->x, s));
+    QH_E(launch_embed(p->embd, p->tok, p->pos, feedback ? nullptr : p->pinned, c.vocab_size, c.max_seq_len,
+                      c.dim, p->x, s));
     GemvDecode dec;
     dec.pos = p->pos;
     dec.cos_tab = p->cos_tab;
@@ -708,8 +706,7 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
     const size_t o_pm = carve((size_t)cfg.n_heads * nch * 4), o_ps = carve((size_t)cfg.n_heads * nch * 4);
     const size_t o_op = carve(nch * cfg.n_heads * hd * 4);
     const size_t o_ct = carve(tab * 4), o_st = carve(tab * 4);
-    const size_t o_tok = carve(4), o_pos = carve(4), o_lp = carve(4), o_hn = carve(4);
-    const size_t o_hist = carve((size_t)p->hist_cap * 4);
+    const size_t o_tok = carve(4), o_pos = carve(4), o_hn = carve(4), o_hist = carve((size_t)p->hist_cap * 4);
     const size_t o_aw = carve(argmax_workspace_bytes(cfg.vocab_size));
     const size_t o_ap = carve((size_t)2 * kGemvAmaxMaxParts * 4);
     hipError_t e = hipMalloc(&p->arena, bytes);
@@ -723,8 +720,7 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
         plan_destroy(st);
         return Q_ERR_ALLOC_FAILED;
     }
-    p->pinned[2] = 0;  // (sources of small copies)
-    p->pinned[3] = 1;
+    p->pinned[2] = 0;
     p->arena_bytes = bytes;
     uint8_t* A = p->arena;
     p->x = reinterpret_cast<float*>(A + o_x);
@@ -744,7 +740,6 @@ q_error_code llama_build_graph(q_context* __restrict__ ctx, q_llama_model* __res
     p->sin_tab = reinterpret_cast<float*>(A + o_st);
     p->tok = reinterpret_cast<uint32_t*>(A + o_tok);
     p->pos = reinterpret_cast<uint32_t*>(A + o_pos);
-    p->looped = reinterpret_cast<uint32_t*>(A + o_lp);
     p->hist_n = reinterpret_cast<uint32_t*>(A + o_hn);
     p->hist = reinterpret_cast<uint32_t*>(A + o_hist);
     p->amax_ws = reinterpret_cast<float*>(A + o_aw);
@@ -823,10 +818,6 @@ q_error_code llama_forward(q_llama_model* __restrict__ model, q_context* __restr
         p->pinned[0] = tokens[0];
         p->pinned[1] = pos;
         // (the step's embedding launch reads them from there)
-        if (p->loop_set) {
-            QH_TRY(hipMemcpyAsync(p->looped, &p->pinned[2], 4, hipMemcpyHostToDevice, p->stream));
-            p->loop_set = false;
-        }
         QH_TRY(hipGraphLaunch(p->step_graph, p->stream));
     } else {
         QH_TRY_CODE(prefill_alloc(p));
@@ -969,11 +960,10 @@ q_error_code qh_llama_generate_sampled(q_llama_model* model, q_context* ctx, uin
     sp.top_p = top_p;
     QH_TRY(hipStreamSynchronize(p->stream));
     p->pinned[0] = token;
-    p->pinned[1] = pos;
-    QH_TRY(hipMemcpyAsync(p->looped, &p->pinned[3], 4, hipMemcpyHostToDevice, p->stream));
-    p->loop_set = true;
+    p->pinned[1] = kOnDevice;  // (the step graph takes them from the device)
+    p->pinned[3] = pos;
     QH_TRY(hipMemcpyAsync(p->tok, &p->pinned[0], 4, hipMemcpyHostToDevice, p->stream));
-    QH_TRY(hipMemcpyAsync(p->pos, &p->pinned[1], 4, hipMemcpyHostToDevice, p->stream));
+    QH_TRY(hipMemcpyAsync(p->pos, &p->pinned[3], 4, hipMemcpyHostToDevice, p->stream));
     QH_TRY(hipMemcpyAsync(p->hist_n, &p->pinned[2], 4, hipMemcpyHostToDevice, p->stream));
     hipEvent_t e0, e1;
     QH_TRY(hipEventCreate(&e0));

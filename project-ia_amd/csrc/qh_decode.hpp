@@ -32,11 +32,11 @@ size_t attention_n_chunks(uint32_t max_seq);
 hipError_t launch_swiglu_prep(const float* g, const float* u, uint32_t N, float* m_out, uint4* xd, hipStream_t s);
 // host: null (token and position are in device memory), or two words of pinned
 // memory (token, position; 8-byte aligned) that the launch reads and stores to
-// tok and pos while *looped (device) is 0.
+// tok and pos, unless the second is kOnDevice (no position: they are below it).
 // A position outside 0 .. max_seq-1 is stored as the nearest one inside.
-hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host,
-                        const uint32_t* looped, uint32_t vocab, uint32_t max_seq, uint32_t dim, float* x,
-                        hipStream_t s);
+constexpr uint32_t kOnDevice = 0xFFFFFFFFu;
+hipError_t launch_embed(const float* embd, uint32_t* tok, uint32_t* pos, const uint32_t* host, uint32_t vocab,
+                        uint32_t max_seq, uint32_t dim, float* x, hipStream_t s);
 // n device floats to pinned host memory.
 hipError_t launch_to_host(const float* src, float* dst, uint32_t n, hipStream_t s);
 
