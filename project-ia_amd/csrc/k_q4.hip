@@ -109,20 +109,24 @@ __global__ __launch_bounds__(256) void k_dequant(const uint32_t* __restrict__ bl
     }
 }
 
-// The stores write through the L2, which spares its write-backs: the data is
+// The stores write through the L2, which spares its write-backs: the output is
 // in the 256 MB memory-side cache when the kernel that reads it next comes.
-// Where blocks (20 bytes) and output (128) together pass that cache, they also
-// carry the non-temporal hint.  us alone / with a reading kernel behind / with
-// one that reads and writes:
-//   output   plain stores         write through        and non-temporal
-//     8 MB    3.4   13.1   12.3    3.5   12.6   12.1    3.4   12.9   13.1
-//    34 MB    8.2   28.2   28.2    7.0   28.1   27.4    7.3   30.7   33.2
-//    64 MB   12.6   31.1   43.2   10.5   30.8   42.6   11.5   33.7   52.8
-//   128 MB   23.8   49.8   81.4   19.6   49.4   78.9   22.6   53.8   96.3
-//   200 MB   35.7   73.6  159.7   31.7   72.8  157.6   34.8   83.0  160.6
-//   230 MB   45.5   99.7  187.3   43.5   96.5  186.0   39.4   91.8  184.7
-//   300 MB   66.2  152.2  240.0   63.5  150.5  238.1   53.5  134.8  239.9
-constexpr uint64_t kDequantNtBlocks = (256ull << 20) / (20 + 128);
+// Where blocks (20 bytes) and output (128) together pass half of that cache,
+// much of it would be gone by then, or push out what is still to be written:
+// there they also carry the non-temporal hint.  us alone / with a reading
+// kernel behind / with one that reads and writes, over 700 MB of outputs in
+// turn (8 and 20 MB: plain stores instead of the hint):
+//   output   non-temporal            write through
+//     8 MB     4.0   11.6    9.1       3.7   11.4    8.9
+//    20 MB     6.4   15.7   16.3       5.5   15.1   15.7
+//    34 MB     7.4   23.5   28.6       8.2   21.5   23.6
+//    64 MB    13.0   34.4   50.8      14.6   30.4   41.0
+//    96 MB    18.4   47.4   74.2      21.3   44.6   65.1
+//   128 MB    24.0   58.6  101.4      28.3   62.4   81.8
+//   200 MB    36.9   89.6  160.3      43.2   97.8  153.7
+// (On one output over and over, which never leaves the cache, writing through
+// alone is the faster one up to 200 MB, also alone: 64 MB 10.5 against 11.5.)
+constexpr uint64_t kDequantNtBlocks = (128ull << 20) / (20 + 128);
 
 hipError_t launch_dequant(const uint8_t* blocks, float* out, uint64_t n_blocks, hipStream_t s) {
     if (n_blocks == 0) return hipSuccess;

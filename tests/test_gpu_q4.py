@@ -93,7 +93,8 @@ def test_dequant_device_bitexact_random_and_adversarial(qa):
 
 # Wave and workgroup edges (64 and 256 blocks) and both sides of the size past
 # which the stores are non-temporal.
-@pytest.mark.parametrize("nb", [1, 2, 63, 64, 65, 255, 256, 257, 1000, 262144, 262145, 262209, 1813752, 1813753, 1813817])
+@pytest.mark.parametrize("nb", [1, 2, 63, 64, 65, 255, 256, 257, 1000, 262144, 262145, 262209, 906876, 906877, 906941, 1813752,
+                                1813753, 1813817])
 def test_dequant_block_counts_bitexact(qa, nb):
     rng = orc.rng_for(103, nb)
     blob = orc.gen_q4(nb, 32, rng).reshape(-1)
